@@ -69,4 +69,46 @@ __device__ inline u64 block_excl_scan(u64 v, u64 *tmp, u64 &total) {
     return r;
 }
 
+// ---------------------------------------------------------------------------
+// A step driven from the device (qd_k_lean.hpp): its sizes and layout, read
+// by each kernel when it starts.
+// ---------------------------------------------------------------------------
+enum : u32 {
+    LEAN_ERR = 1u,      // an invalid object, or a graph beyond the fast kernels' 64 nodes
+    LEAN_EMPTY = 2u,    // no candidates
+    LEAN_BIG = 4u,      // more candidates than there is room for
+    LEAN_BUCKET = 8u,   // a bucket that the main dedup kernel hands back
+    LEAN_SPILL = 32u,   // a bucket beyond its capacity (ERR_SPILL1's bit)
+    LEAN_SELECT = 64u   // more tied keys than one block takes, or a subnormal threshold
+};
+// Kernels that can stop the step, in launch order.  Each sets its own word,
+// and a kernel looks only at the words of the kernels before it, so that
+// every thread of it sees the same.
+enum : int { LEAN_SCAN, LEAN_GENERATE, LEAN_LEVEL2, LEAN_DEDUP, LEAN_HIST, LEAN_FIRST, LEAN_FINISH, LEAN_EMIT };
+struct LeanPlan {
+    u64 C, items;      // candidates, work items
+    u64 cap1, cap2;    // bucket capacities of the first and second radix pass
+    u64 counters[8];   // the dedup's: [0] uniques, [5] and [6] buckets handed back
+    u64 r1, r2;        // select: keys still to take after the first and second digit
+    u64 ns;            // select: keys that tie after the second digit
+    u64 K, bytes;      // survivors and their padded bytes
+    u32 b1, b2;        // bits of the radix passes
+    u32 d1;            // select: the first digit
+    u32 ticket[3];     // next tiles of the look-back kernels
+    u32 stop[LEAN_EMIT];  // LEAN_* by kernel (the dedup's: counters 5 and 6)
+};
+// What the last kernel reports to the host (pinned memory).
+struct LeanReport {
+    u64 U, K, bytes;
+    double total;
+    u32 stop, fits, b1, b2;
+};
+// The reasons to stop that the kernels before `stage` gave.
+__device__ inline u32 lean_stopped(const LeanPlan *lp, int stage) {
+    u32 w = 0;
+    for (int i = 0; i < stage; ++i) w |= lp->stop[i];
+    if (stage > LEAN_DEDUP && (lp->counters[5] | lp->counters[6])) w |= LEAN_BUCKET;
+    return w;
+}
+
 }  // namespace qd

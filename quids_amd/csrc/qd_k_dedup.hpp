@@ -368,7 +368,18 @@ constexpr int kWideCandBits = 40;
 template <int T, int CAP, int TS>
 __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const u64 *woff, u64 nbk, u32 L, double tol,
                                              u64 *UH, u64 *UR, double2 *UM, u32 *UK, u64 *counters, u64 *nhist,
-                                             u64 *biglist, u64 *redolist) {
+                                             u64 *biglist, u64 *redolist, LeanPlan *lp, const Entry *E2) {
+    if (lp) {  // a step driven from the device: the buckets of E, or of E2 after a second pass
+        if (lean_stopped(lp, LEAN_DEDUP)) return;
+        L = lp->b1 + lp->b2;
+        nbk = 1ull << L;
+        rstride = lp->b2 ? lp->cap2 : lp->cap1;
+        if (lp->b2) E = E2;
+        counters = lp->counters;
+        const u64 C = lp->C;  // UH / UR / UM: C slots of one buffer
+        UR = UH + C;
+        UM = reinterpret_cast<double2 *>(UR + C);
+    }
     constexpr int PER = CAP / T;
     constexpr u32 kNil = 0xFFFFFFFFu;  // empty member list (any value >= CAP ends a list)
     static_assert(CAP <= 4096 && TS <= 4096, "packed wide keys hold 12-bit slots and entries");

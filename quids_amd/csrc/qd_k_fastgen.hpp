@@ -36,6 +36,14 @@ enum : u8 { PD_FS = 1, PD_LM = 2, PD_HMLZ = 4 };
 // step then runs on the generic per-byte kernels).
 constexpr u32 ERR_WIDE = 8u;
 
+// Child sizes of split_merge without its walk: by how many bytes each
+// decision of a parent, taken, makes the child larger than the parent
+// (a split: one node more, and its halves' names for its own; a merge: one
+// node less, and the merged name for the two), at delta[sm_delta_base + d]
+// for decision d.  A valid graph of n nodes spans at least 20 n bytes, so the
+// parents' runs do not overlap.
+QD_HD u64 sm_delta_base(u64 begin) { return begin / 20; }
+
 // Descriptor of parent p, computed by a segment of SEG lanes (one lane per
 // node: SEG = 64, or 32 / 16 when two / four parents share a wavefront; the
 // segment's lanes are active together).  have: the segment
@@ -43,7 +51,7 @@ constexpr u32 ERR_WIDE = 8u;
 // NC_ONLY: the child count alone (nc; D, wi and tab untouched).
 template <int KIND, int SEG, bool NC_ONLY = false>
 __device__ inline void prep_parent(const Parents &P, u64 p, bool have, const u64 *keep, PDesc *D, u32 *nc, u32 *wi,
-                                   u64 *tab, u32 &local_max, u32 *err) {
+                                   u64 *tab, i32 *delta, u32 &local_max, u32 *err) {
     const u32 lane = threadIdx.x & (kWave - 1);
     const u32 sl = lane & (SEG - 1);      // node of this lane
     const u32 sbase = lane & ~(SEG - 1);  // first lane of the segment
@@ -126,6 +134,18 @@ __device__ inline void prep_parent(const Parents &P, u64 p, bool have, const u64
             t[1] = split ? split_left_hash(g, b) : merge_hash(g, b, g.name_begin(sl + 1 < n ? sl + 1 : 0));
             t[2] = split ? split_right_hash(g, b) : 0;
         }
+        if (!NC_ONLY && delta && in) {  // see sm_delta_base
+            const u32 dn = (lmg ? 1u : 0u) + u32(__popcll(d.dmask & ((1ull << sl) - 1)));
+            const u32 b = g.name_begin(sl), m = g.name_begin(sl + 1) - b;
+            i32 *dt = delta + sm_delta_base(P.begin[p]);
+            if (split) {
+                dt[dn] = 4 + 16 * (g.sub_type(b) >= 0 ? -1 : i32(m) + 2);
+            } else if (merge || (lmg && sl + 1 == n)) {
+                const u32 nx = sl + 1 < n ? sl + 1 : 0, bb = g.name_begin(nx);
+                const i32 mb = i32(g.name_begin(nx + 1) - bb);
+                dt[merge ? dn : 0u] = -4 + 16 * (merge_collapses(g, b, bb) ? -(1 + mb) : 1);
+            }
+        }
         local_max = max(local_max, 4 * sz);
     } else {
         const bool coin = KIND == QD_RULE_QCGD_COIN;
@@ -156,7 +176,7 @@ __device__ inline void prep_parent(const Parents &P, u64 p, bool have, const u64
 // one after the other on the whole wavefront.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_prep_fast(Parents P, const u64 *keep, PDesc *D, u32 *nc, u32 *wi, u64 *tab,
-                                                   u32 *maxsz, u32 *err) {
+                                                   i32 *delta, u32 *maxsz, u32 *err) {
     const u32 lane = threadIdx.x & (kWave - 1);
     const u64 nwaves = u64(gridDim.x) * (blockDim.x / kWave);
     u32 local_max = 0;
@@ -165,15 +185,15 @@ __global__ __launch_bounds__(256) void k_prep_fast(Parents P, const u64 *keep, P
         if (lane < 4 && p0 + lane < P.n && P.size[p0 + lane] >= 4) nq = ld16(P.obj + P.begin[p0 + lane]);
         if (__ballot(nq > 16) == 0) {
             const u64 p = p0 + lane / 16;
-            prep_parent<KIND, 16>(P, p, p < P.n, keep, D, nc, wi, tab, local_max, err);
+            prep_parent<KIND, 16>(P, p, p < P.n, keep, D, nc, wi, tab, delta, local_max, err);
         } else if (__ballot(nq > 32) == 0) {
             for (u32 h = 0; h < 2; ++h) {
                 const u64 p = p0 + 2 * h + lane / 32;
-                prep_parent<KIND, 32>(P, p, p < P.n, keep, D, nc, wi, tab, local_max, err);
+                prep_parent<KIND, 32>(P, p, p < P.n, keep, D, nc, wi, tab, delta, local_max, err);
             }
         } else {
             for (u32 q = 0; q < 4; ++q)
-                prep_parent<KIND, kWave>(P, p0 + q, p0 + q < P.n, keep, D, nc, wi, tab, local_max, err);
+                prep_parent<KIND, kWave>(P, p0 + q, p0 + q < P.n, keep, D, nc, wi, tab, delta, local_max, err);
         }
     }
     for (int off = kWave / 2; off > 0; off >>= 1) local_max = max(local_max, (u32)__shfl_xor(int(local_max), off, kWave));
@@ -194,16 +214,16 @@ __global__ __launch_bounds__(256) void k_num_child_fast(Parents P, u32 *nc, u32 
         if (lane < 4 && p0 + lane < P.n && P.size[p0 + lane] >= 4) nq = ld16(P.obj + P.begin[p0 + lane]);
         if (__ballot(nq > 16) == 0) {
             const u64 p = p0 + lane / 16;
-            prep_parent<KIND, 16, true>(P, p, p < P.n, nullptr, nullptr, nc, nullptr, nullptr, local_max, err);
+            prep_parent<KIND, 16, true>(P, p, p < P.n, nullptr, nullptr, nc, nullptr, nullptr, nullptr, local_max, err);
         } else if (__ballot(nq > 32) == 0) {
             for (u32 h = 0; h < 2; ++h) {
                 const u64 p = p0 + 2 * h + lane / 32;
-                prep_parent<KIND, 32, true>(P, p, p < P.n, nullptr, nullptr, nc, nullptr, nullptr, local_max, err);
+                prep_parent<KIND, 32, true>(P, p, p < P.n, nullptr, nullptr, nc, nullptr, nullptr, nullptr, local_max, err);
             }
         } else {
             for (u32 q = 0; q < 4; ++q)
                 prep_parent<KIND, kWave, true>(P, p0 + q, p0 + q < P.n, nullptr, nullptr, nc, nullptr, nullptr,
-                                               local_max, err);
+                                               nullptr, local_max, err);
         }
     }
 }

@@ -68,6 +68,12 @@ __global__ __launch_bounds__(256) void k_child_size(Parents P, const u64 *cb, qd
     }
 }
 
+// Whether the survivors of a step driven from the device have room in the
+// output state (capk objects, capb bytes).
+__device__ inline bool lean_fits(const LeanPlan *lp, u64 capk, u64 capb) {
+    return !lean_stopped(lp, LEAN_EMIT) && lp->K <= capk && lp->bytes <= capb;
+}
+
 // One wavefront per survivor, everything lane-parallel:
 //  * erase_create / coin / hadamard: the child is the parent with some
 //    particle (qubit) bytes flipped -- one coalesced copy, the flips applied
@@ -175,7 +181,11 @@ __device__ inline void populate_flip_one(const Parents &P, const u64 *cb, const 
 template <int KIND>
 __global__ __launch_bounds__(256) void k_populate_flip(Parents P, const u64 *cb, qd_rule rule, const u64 *orep,
                                                        const u64 *opar, u64 K, const u64 *obegin, const u32 *osize,
-                                                       u8 *oobj) {
+                                                       u8 *oobj, const LeanPlan *lp, u64 capb) {
+    if (lp) {  // a step driven from the device: K objects of room, capb bytes
+        if (!lean_fits(lp, K, capb)) return;
+        K = lp->K;
+    }
     const u32 lane = threadIdx.x & (kWave - 1);
     const u64 wave = (u64(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
     const u64 nwaves = u64(gridDim.x) * blockDim.x / kWave;
@@ -212,7 +222,11 @@ __device__ inline u32 seg_excl_sum(u32 v, u32 &total) {
 
 __global__ __launch_bounds__(kWave) void k_populate_sm(Parents P, const u64 *cb, qd_rule rule, const u64 *orep,
                                                     const u64 *opar, u64 K, const u64 *obegin, const u32 *osize,
-                                                    u8 *oobj) {
+                                                    u8 *oobj, const LeanPlan *lp, u64 capb) {
+    if (lp) {  // as in k_populate_flip
+        if (!lean_fits(lp, K, capb)) return;
+        K = lp->K;
+    }
     __shared__ __align__(16) u8 pbuf[kPopSegs][kPopParent];
     __shared__ __align__(16) u8 cbuf[kPopSegs][kPopChild];
     __shared__ u8 ckind[kPopSegs][kPopNodes], cl[kPopSegs][kPopNodes], cr[kPopSegs][kPopNodes];
@@ -372,12 +386,11 @@ __global__ __launch_bounds__(kWave) void k_populate_sm(Parents P, const u64 *cb,
 constexpr int kSumThreads = 256;
 constexpr int kSumChunk = 2048;
 
-// One block per chunk of 2048 values: lane t sums t, t+256, ..., t+1792 in
-// order, then a halving tree s[t] += s[t+stride], stride = 128 .. 1.
-__global__ __launch_bounds__(kSumThreads) void k_sum_chunks(const double2 *mag, const double *vals, u64 n,
-                                                            double *out) {
-    __shared__ double s[kSumThreads];
-    const u64 base = u64(blockIdx.x) * kSumChunk;
+// Chunk `ch` of 2048 of the n values (|m|^2, or vals when mag is null), by
+// one block: lane t sums t, t+256, ..., t+1792 in order, then a halving tree
+// s[t] += s[t+stride], stride = 128 .. 1.  Every thread gets the sum.
+__device__ inline double sum_chunk(const double2 *mag, const double *vals, u64 n, u64 ch, double *s) {
+    const u64 base = ch * kSumChunk;
     double a = 0.0;
     for (int j = 0; j < kSumChunk / kSumThreads; ++j) {
         const u64 i = base + threadIdx.x + u64(kSumThreads) * j;
@@ -398,7 +411,14 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_chunks(const double2 *mag, 
         if (threadIdx.x < stride) s[threadIdx.x] = s[threadIdx.x] + s[threadIdx.x + stride];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = s[0];
+    return s[0];
+}
+
+__global__ __launch_bounds__(kSumThreads) void k_sum_chunks(const double2 *mag, const double *vals, u64 n,
+                                                            double *out) {
+    __shared__ double s[kSumThreads];
+    const double t = sum_chunk(mag, vals, n, blockIdx.x, s);
+    if (threadIdx.x == 0) out[blockIdx.x] = t;
 }
 
 __global__ __launch_bounds__(256) void k_scale(double2 *mag, u64 n, double f) {

@@ -56,6 +56,7 @@
 #include "qd_k_batch.hpp"
 #include "qd_k_range.hpp"
 #include "qd_k_user.hpp"
+#include "qd_k_lean.hpp"
 
 using namespace qd;
 
@@ -204,6 +205,8 @@ constexpr u64 kNoAllocDoubles = kNoAllocMaxObjects + 2 * ((kNoAllocMaxObjects + 
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
 constexpr u64 kHostN = 8191;  // slot of the pinned area that stages a value for the device
+constexpr u64 kHostScan = 7960;  // reports of the device-driven step: the scan's, the last kernel's
+constexpr u64 kHostLean = 7968;
 constexpr u64 kHostSegLoop = 8000;  // first of the slots that stage the batched select loop's state
 constexpr u64 kHostSelLoop = 8064;  // first of the slots that stage the select loop's state
 
@@ -245,6 +248,7 @@ struct qd_ctx {
                                                 // children's slice tags, per-block bucket counts, group offsets,
     DBuf rcnt, abuf;                            // region counts, a group's merged first-level buckets
     DBuf slab;  // one allocation kept across hash-range steps, carved into their big buffers (views)
+    DBuf lean, ctab, delta;  // the device-driven step: plan, chunks' first parents, child size differences
     DBuf usize, uscr;  // user rules: every candidate's child size, the generate's child bytes
     // output buffers of batched chunks (objects, begin, size, mag per chunk),
     // kept between calls
@@ -261,7 +265,7 @@ struct qd_ctx {
                 &biglist, &redolist, &bigsoff, &bigkey, &bigcand, &bigmag, &bigseg, &pdesc, &wi, &wb, &cpar, &opar, &ebuf2, &cnt2, &slist, &ukey, &selloop, &segloop, &bsoff, &bscnt,
                 &adjk, &adjv, &adjg, &adjd, &adjp, &adjw, &bseg, &boseg, &brules, &bsinst, &bcount, &bsel, &btrunc,
                 &blist, &bcur, &btile, &bhist, &bkseg, &bchunk, &bcsum, &btot, &pool0, &pool1, &pwpre, &blist2, &mw, &rpart[0], &rpart[1], &rpart[2],
-                &rpart[3], &pk0, &pk1, &tags, &bmat, &goff, &rcnt, &abuf, &slab, &usize, &uscr};
+                &rpart[3], &pk0, &pk1, &tags, &bmat, &goff, &rcnt, &abuf, &slab, &usize, &uscr, &lean, &ctab, &delta};
     }
     void set_names() {
         static const char *const names[] = {
@@ -271,10 +275,11 @@ struct qd_ctx {
             "slist", "ukey", "selloop", "segloop", "bsoff", "bscnt", "adjk", "adjv", "adjg", "adjd", "adjp", "adjw",
             "bseg", "boseg", "brules", "bsinst", "bcount", "bsel", "btrunc", "blist", "bcur", "btile", "bhist",
             "bkseg", "bchunk", "bcsum", "btot", "pool0", "pool1", "pwpre", "blist2", "mw", "rpart0", "rpart1",
-            "rpart2", "rpart3", "pk0", "pk1", "tags", "bmat", "goff", "rcnt", "abuf", "slab", "usize", "uscr"};
+            "rpart2", "rpart3", "pk0", "pk1", "tags", "bmat", "goff", "rcnt", "abuf", "slab", "usize", "uscr", "lean",
+            "ctab", "delta"};
         std::vector<DBuf *> v = all_named();
         constexpr size_t kNames = sizeof(names) / sizeof(names[0]);
-        static_assert(kNames == 81, "one name per buffer");
+        static_assert(kNames == 84, "one name per buffer");
         for (size_t i = 0; i < v.size() && i < kNames; ++i) v[i]->name = names[i];
     }
 };
@@ -539,6 +544,15 @@ static int select_loop(qd_ctx *ctx, SelItem *S0, SelItem *S1, u64 ns, u64 r, u32
     }
     QD_TRY(ctx->selloop.ensure(sizeof(SelLoop)));
     SelLoop *dL = ctx->selloop.as<SelLoop>();
+    if (ns <= kSelFinish && !ctx->tune.eager_select) {
+        hipLaunchKernelGGL(k_sel_finish, dim3(1), dim3(1024), 0, s, (const SelItem *)S0, u32(ns), r, pos, UR, bitmap,
+                           sbm, &dL->state);
+        QD_HIP(hipGetLastError());
+        QD_TRY(sync_read(ctx, &dL->state, sizeof(u32), ctx->host));
+        if (*reinterpret_cast<const u32 *>(ctx->host) != 1)
+            return fail(QD_ERR_HIP, "select did not converge (duplicate keys)");
+        return QD_OK;
+    }
     SelLoop h{};
     h.items[0] = S0;
     h.items[1] = S1;
@@ -758,7 +772,7 @@ static int dedup_phase(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *woff
     auto run_dedup = [&](auto kern, int threads) -> int {
         hipLaunchKernelGGL(kern, dim3(resident(kern, threads, nbk)), dim3(threads), 0, s, D, rstride, woff, nbk, L,
                            tol, UH, UR, UM, UK, counters, ctx->nhist.as<u64>(), ctx->biglist.as<u64>(),
-                           ctx->redolist.as<u64>());
+                           ctx->redolist.as<u64>(), (LeanPlan *)nullptr, (const Entry *)nullptr);
         QD_HIP(hipGetLastError());
         return QD_OK;
     };
@@ -866,7 +880,7 @@ static int partition_dedup(qd_ctx *ctx, const u64 *H0, const double2 *M0, const 
             (void)hipDeviceGetAttribute(&ncu2, hipDeviceAttributeMultiprocessorCount, ctx->device);
             const unsigned g2 = unsigned(std::min<u64>(nb1, std::max(ncu2 / 2, 1)));
             hipLaunchKernelGGL(k_level2_fixed, dim3(g2), dim3(1024), 0, s, (const Entry *)E1, in_stride,
-                               ctx->off1.as<u64>(), nb1, b1, b2, cap2, E2, ctx->cnt2.as<u64>(), errw);
+                               ctx->off1.as<u64>(), nb1, b1, b2, cap2, E2, ctx->cnt2.as<u64>(), errw, (LeanPlan *)nullptr);
             QD_HIP(hipGetLastError());
             QD_TRY(run_scan(ctx, LoadU64{ctx->cnt2.as<u64>()}, nb, ctx->off2.as<u64>()));
             QD_TRY(sync_read(ctx, errw, sizeof(u32), &ew));
@@ -922,11 +936,12 @@ static int populate_out(qd_ctx *ctx, const Parents &P, const qd_rule &rule, cons
         hipLaunchKernelGGL(k_populate_sm, dim3(unsigned(std::min<u64>((K + kPopSegs - 1) / kPopSegs, 65536))),
                            dim3(kWave), 0, s, P,
                            ctx->cb.as<u64>(), rule, orep, (const u64 *)ctx->opar.as<u64>(), K, out->begin.as<u64>(),
-                           out->size.as<u32>(), out->objects.as<u8>());
+                           out->size.as<u32>(), out->objects.as<u8>(), (const LeanPlan *)nullptr, u64(0));
     else
         hipLaunchKernelGGL(k_populate_flip<KIND>, dim3(unsigned(std::min<u64>((K + 7) / 8, 65536))), dim3(256), 0, s,
                            P, ctx->cb.as<u64>(), rule, orep, (const u64 *)ctx->opar.as<u64>(), K,
-                           out->begin.as<u64>(), out->size.as<u32>(), out->objects.as<u8>());
+                           out->begin.as<u64>(), out->size.as<u32>(), out->objects.as<u8>(),
+                           (const LeanPlan *)nullptr, u64(0));
     QD_HIP(hipGetLastError());
     out->n = K;
     out->bytes = bytes;
@@ -1334,7 +1349,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
         QD_TRY(carve(ctx->tab, tab_bytes));
         hipLaunchKernelGGL(k_prep_fast<KIND>, dim3(grid_for(N, 16, 65536)), dim3(256), 0, s, P, keep,
                            ctx->pdesc.as<PDesc>(), ctx->nc.as<u32>(), ctx->wi.as<u32>(), ctx->tab.as<u64>(),
-                           reinterpret_cast<u32 *>(counters + 3), errw);
+                           (i32 *)nullptr, reinterpret_cast<u32 *>(counters + 3), errw);
         QD_HIP(hipGetLastError());
     }
     QD_TRY(carve(ctx->tags, std::max<u64>(u64(T) * pstride, 8)));
@@ -1661,7 +1676,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
                     (void)hipDeviceGetAttribute(&ncu2, hipDeviceAttributeMultiprocessorCount, ctx->device);
                     const unsigned g2 = unsigned(std::min<u64>(gbk, std::max(ncu2 / 2, 1)));
                     hipLaunchKernelGGL(k_level2_fixed, dim3(g2), dim3(1024), 0, s, gin, u64(0), go, gbk, b1, b2, cap2,
-                                       E2, ctx->cnt2.as<u64>(), errw);
+                                       E2, ctx->cnt2.as<u64>(), errw, (LeanPlan *)nullptr);
                     QD_HIP(hipGetLastError());
                     QD_TRY(run_scan(ctx, LoadU64{ctx->cnt2.as<u64>()}, nb2g, ctx->off2.as<u64>()));
                     u32 ew2 = 0;
@@ -2000,6 +2015,194 @@ static int plain_select(qd_ctx *ctx, u64 C, u64 U, u64 max_obj, const SelKey &sk
     return select_topk(ctx, UH, UR, UM, UK, C, max_obj, h, bitmap, sbm, sk);
 }
 
+// ===========================================================================
+// the step driven from the device (qd_k_lean.hpp)
+// ===========================================================================
+constexpr u64 kLeanSpec = 1ull << 18;     // candidates there is room for before their number is known
+constexpr u64 kLeanSpecParents = 2048;    // ... for steps of at most so many parents
+constexpr u64 kLeanChildMax = 1ull << 20; // candidates generated one child per lane; beyond, by work items
+constexpr u64 kLeanTab = kLeanMax / kLeanChunk + 1;
+
+// The plan and the arrays cleared with it, in u64 words.
+struct LeanArea {
+    u64 cnt1, nhist, hist2, emit_desc, emit_tiles, scan_desc, scan_tiles, words;
+    explicit LeanArea(u64 N) {
+        cnt1 = (sizeof(LeanPlan) + 7) / 8;
+        nhist = cnt1 + 256;
+        hist2 = nhist + kHistBins;
+        emit_desc = hist2 + kHistBins;
+        emit_tiles = kLeanMax / kEmitTile;
+        scan_desc = emit_desc + 2 * emit_tiles;
+        scan_tiles = (N + kScanTile - 1) / kScanTile;
+        words = scan_desc + 2 * scan_tiles;
+    }
+};
+
+// How a device-driven tail ended.
+struct LeanEnd {
+    bool done = false;  // the output state is complete
+    u32 stop = 0;       // else why not (LEAN_*)
+    u64 U = 0;
+};
+
+// The device-driven step takes plain |m|^2 keys and the default layout; a
+// phase hook is called between phases that it does not wait between.
+static bool lean_allowed(qd_ctx *ctx, const SelKey &sk) {
+    const qd_tuning &t = ctx->tune;
+    return !sk.prob && !ctx->hook && !t.generic_path && !t.split_generate && !t.eager_select &&
+           t.dedup_bucket_target == 512 && t.first_pass_bits == 8 && t.dedup_cap == 1024;
+}
+
+// Everything after the parents' scan, for at most `room` candidates: C of
+// them when the host knows (C != 0), else what the scan found.  One wait, at
+// the end; a second one when the output state had to grow.
+template <int KIND>
+static int lean_tail(qd_ctx *ctx, const Parents &P, const qd_rule &rule, const LeanArea &la, u64 room, u64 C,
+                     u64 nitems, u64 max_obj, const qd_params &prm, qd_state *out, qd_step_stats &st, LeanEnd &le) {
+    hipStream_t s = ctx->stream;
+    u64 *a = ctx->lean.as<u64>();
+    LeanPlan *lp = reinterpret_cast<LeanPlan *>(a);
+    if (le.stop & LEAN_BIG) hipLaunchKernelGGL(k_lean_room, dim3(1), dim3(64), 0, s, lp);
+    le = LeanEnd{};
+    // room: one bucket pass of 2^8 x cap1 entries (lean_layout grows with C
+    // there), sub-buckets of at most 1024 entries for 240 candidates
+    u32 b1, b2;
+    u64 cap1, cap2;
+    lean_layout(room, b1, b2, cap1, cap2);
+    const u64 bound = std::min(max_obj, room);  // survivors
+    const bool two = b2 != 0, keys = max_obj < room;
+    QD_TRY(ensure_relieved(ctx, ctx->ebuf0, room * 32));
+    QD_TRY(ensure_relieved(ctx, ctx->ebuf1, std::max<u64>(256 * std::max<u64>(cap1, 1024), room) * sizeof(Entry)));
+    if (two) QD_TRY(ensure_relieved(ctx, ctx->ebuf2, (room * 9 / 2 + 4096) * sizeof(Entry)));
+    if (two) QD_TRY(ensure_relieved(ctx, ctx->cnt2, (room / 240 + 256) * sizeof(u64)));
+    QD_TRY(ensure_relieved(ctx, ctx->off2, (room / 240 + 258) * sizeof(u64)));
+    QD_TRY(ensure_relieved(ctx, ctx->ukey, (room + 4) * sizeof(u32)));
+    QD_TRY(ctx->biglist.ensure((room / 1024 + 2) * sizeof(u64)));
+    QD_TRY(ctx->redolist.ensure((room / 240 + 258) * sizeof(u64)));
+    QD_TRY(ctx->sel0.ensure(kSelFinish * sizeof(SelItem)));
+    QD_TRY(ensure_relieved(ctx, ctx->keys, std::max<u64>(bound, 1) * sizeof(u64)));
+    QD_TRY(ensure_relieved(ctx, ctx->opar, std::max<u64>(bound, 1) * sizeof(u64)));
+    QD_TRY(ctx->chunks.ensure(2 * sum_scratch_half(bound) * sizeof(double)));
+    u64 *UH = ctx->ebuf0.as<u64>();  // (the kernels place UR and UM after C of them)
+    Entry *E1 = ctx->ebuf1.as<Entry>(), *E2 = two ? ctx->ebuf2.as<Entry>() : E1;
+    u32 *UK = keys ? ctx->ukey.as<u32>() : nullptr;
+    u32 *slotof = ctx->ebuf1.as<u32>();  // (after the dedup has read its entries)
+    u64 *nhist = a + la.nhist, *hist2 = a + la.hist2, *cnt1 = a + la.cnt1;
+    u64 *cnt2 = two ? ctx->cnt2.as<u64>() : cnt1;
+    const u64 *cb = ctx->cb.as<u64>(), *ctab = ctx->ctab.as<u64>();
+    LeanReport *rep = reinterpret_cast<LeanReport *>(ctx->host + kHostLean);
+
+    prof_begin(ctx, QD_PHASE_GENERATE);
+    if (KIND != QD_RULE_HADAMARD && C > kLeanChildMax) {
+        const u64 nchunk = (nitems + kGenThreads - 1) / kGenThreads;
+        QD_TRY(ensure_relieved(ctx, ctx->cpar, nchunk * sizeof(u64)));
+        hipLaunchKernelGGL(k_chunk_parent, dim3(grid_for(nchunk)), dim3(256), 0, s, ctx->wb.as<u64>(), P.n, nchunk,
+                           ctx->cpar.as<u64>());
+        hipLaunchKernelGGL((k_generate_scatter<KIND == QD_RULE_HADAMARD ? QD_RULE_QCGD_COIN : KIND, false>),
+                           dim3(unsigned(std::min<u64>(nchunk, ctx->tune.generate_grid))), dim3(kGenThreads), 0, s,
+                           (const PDesc *)ctx->pdesc.as<PDesc>(), P.mag, cb, (const u64 *)ctx->wb.as<u64>(), P.n,
+                           (const u64 *)ctx->cpar.as<u64>(), (const u64 *)ctx->tab.as<u64>(), P.begin, rule, nitems, b1,
+                           cap1, cnt1, E1, &lp->stop[LEAN_GENERATE], (const qd_rule *)nullptr, (const u64 *)nullptr, 0u,
+                           u64(0));
+    } else {
+        hipLaunchKernelGGL(k_lean_generate<KIND>, dim3(grid_for(room, kLeanChunk, 1024)), dim3(kLeanChunk), 0, s, P,
+                           (const PDesc *)ctx->pdesc.as<PDesc>(), cb, ctab, (const u64 *)ctx->tab.as<u64>(), rule, lp,
+                           cnt1, E1);
+    }
+    QD_HIP(hipGetLastError());
+    prof_end(ctx, QD_PHASE_GENERATE);
+    prof_begin(ctx, QD_PHASE_PARTITION);
+    if (two)
+        hipLaunchKernelGGL(k_level2_fixed, dim3(128), dim3(1024), 0, s, (const Entry *)E1, u64(0), (const u64 *)cnt1,
+                           u64(0), 0u, 0u, u64(0), E2, cnt2, (u32 *)nullptr, lp);
+    hipLaunchKernelGGL(k_lean_bscan, dim3(1), dim3(1024), 0, s, (const u64 *)cnt1, (const u64 *)cnt2,
+                       (const LeanPlan *)lp, ctx->off2.as<u64>());
+    QD_HIP(hipGetLastError());
+    prof_end(ctx, QD_PHASE_PARTITION);
+    prof_begin(ctx, QD_PHASE_DEDUP);
+    hipLaunchKernelGGL((k_dedup<512, 1024, 2048>), dim3(512), dim3(512), 0, s, (const Entry *)E1, u64(0),
+                       (const u64 *)ctx->off2.as<u64>(), u64(0), 0u, prm.tolerance, UH, (u64 *)nullptr,
+                       (double2 *)nullptr, UK, (u64 *)nullptr, nhist, ctx->biglist.as<u64>(), ctx->redolist.as<u64>(),
+                       lp, (const Entry *)E2);
+    QD_HIP(hipGetLastError());
+    prof_end(ctx, QD_PHASE_DEDUP);
+    prof_begin(ctx, QD_PHASE_SELECT);
+    const unsigned gs = grid_for(room, 1024, 1024);
+    hipLaunchKernelGGL(k_lean_hist2, dim3(gs), dim3(256), 0, s, lp, (const u64 *)nhist, (const u32 *)UK, max_obj, hist2,
+                       slotof);
+    hipLaunchKernelGGL(k_lean_first, dim3(gs), dim3(256), 0, s, lp, (const u64 *)hist2, (const u32 *)UK,
+                       (const u64 *)UH, max_obj, ctx->sel0.as<SelItem>(), slotof);
+    if (keys)
+        hipLaunchKernelGGL(k_lean_finish, dim3(1), dim3(1024), 0, s, lp, (const SelItem *)ctx->sel0.as<SelItem>(),
+                           max_obj, (const u64 *)UH, slotof);
+    QD_HIP(hipGetLastError());
+    prof_end(ctx, QD_PHASE_SELECT);
+    for (int attempt = 0;; ++attempt) {
+        // the output's room, as it is; when it is too small it grows to what
+        // the survivors need, and these kernels run again
+        const u64 capk = std::min<u64>(std::min<u64>(out->begin.cap / sizeof(u64) - 1, out->size.cap / sizeof(u32)),
+                                       std::min<u64>(out->mag.cap / sizeof(double2), bound));
+        const u64 capb = out->objects.cap;
+        double *sums = ctx->chunks.as<double>();
+        prof_begin(ctx, QD_PHASE_ORDER);
+        hipLaunchKernelGGL(k_lean_emit<KIND>, dim3(grid_for(room, kEmitTile, 512)), dim3(kEmitThreads), 0, s, P, cb,
+                           ctab, (const i32 *)ctx->delta.as<i32>(), lp, (const u32 *)slotof, (const u64 *)UH,
+                           prm.align_byte_length, capk, a + la.emit_desc, a + la.emit_desc + la.emit_tiles,
+                           ctx->keys.as<u64>(), ctx->opar.as<u64>(), out->size.as<u32>(), out->begin.as<u64>(),
+                           out->mag.as<double2>());
+        QD_HIP(hipGetLastError());
+        prof_end(ctx, QD_PHASE_ORDER);
+        prof_begin(ctx, QD_PHASE_FINALIZE);
+        if (KIND == QD_RULE_QCGD_SPLIT_MERGE)
+            hipLaunchKernelGGL(k_populate_sm, dim3(grid_for(bound, kPopSegs, 8192)), dim3(kWave), 0, s, P, cb, rule,
+                               (const u64 *)ctx->keys.as<u64>(), (const u64 *)ctx->opar.as<u64>(), capk,
+                               (const u64 *)out->begin.as<u64>(), (const u32 *)out->size.as<u32>(),
+                               out->objects.as<u8>(), (const LeanPlan *)lp, capb);
+        else
+            hipLaunchKernelGGL(k_populate_flip<KIND>, dim3(grid_for(bound, 8, 8192)), dim3(256), 0, s, P, cb, rule,
+                               (const u64 *)ctx->keys.as<u64>(), (const u64 *)ctx->opar.as<u64>(), capk,
+                               (const u64 *)out->begin.as<u64>(), (const u32 *)out->size.as<u32>(),
+                               out->objects.as<u8>(), (const LeanPlan *)lp, capb);
+        QD_HIP(hipGetLastError());
+        prof_end(ctx, QD_PHASE_FINALIZE);
+        prof_begin(ctx, QD_PHASE_NORMALIZE);
+        hipLaunchKernelGGL(k_lean_sum, dim3(grid_for(bound, kSumChunk, 512)), dim3(kSumThreads), 0, s,
+                           (const LeanPlan *)lp, capk, capb, (const double2 *)out->mag.as<double2>(), sums);
+        hipLaunchKernelGGL(k_lean_scale, dim3(grid_for(bound, 1024, 1024)), dim3(kSumThreads), 0, s,
+                           (const LeanPlan *)lp, capk, capb, (const double *)sums, out->mag.as<double2>(), rep);
+        QD_HIP(hipGetLastError());
+        prof_end(ctx, QD_PHASE_NORMALIZE);
+        QD_HIP(hipStreamSynchronize(s));
+        prof_collect(ctx);
+        le.stop = rep->stop;
+        le.U = rep->U;
+        if (rep->stop) return QD_OK;
+        if (rep->fits) break;
+        if (attempt) return fail(QD_ERR_HIP, "device-driven step: the output does not fit the room made for it");
+        const u64 K = rep->K, bytes = rep->bytes;
+        QD_TRY(ensure_relieved(ctx, out->begin, (K + 1) * sizeof(u64)));
+        QD_TRY(ensure_relieved(ctx, out->size, std::max<u64>(K, 1) * sizeof(u32)));
+        QD_TRY(ensure_relieved(ctx, out->mag, std::max<u64>(K, 1) * sizeof(double2)));
+        QD_TRY(ensure_relieved(ctx, out->objects, std::max<u64>(bytes, 1)));
+        hipLaunchKernelGGL(k_lean_clear, dim3(32), dim3(256), 0, s, a + la.emit_desc, 2 * la.emit_tiles,
+                           reinterpret_cast<u64 *>(lp->ticket), u64(1));
+        QD_HIP(hipGetLastError());
+    }
+    const u64 K = rep->K;
+    st.num_unique = rep->U;
+    st.num_survivors = K;
+    st.output_bytes = rep->bytes;
+    if (K) {
+        out->n = K;
+        out->bytes = rep->bytes;
+        out->total_proba = rep->total;
+        if (K > u64(kSumChunk) * kSumChunk) QD_TRY(normalize_state(ctx, out));
+        st.total_proba = out->total_proba;
+    }
+    le.done = true;
+    return QD_OK;
+}
+
 template <int KIND, bool BATCH>
 static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, const qd_rule &rule, Batch *bt,
                      qd_state *out, qd_symbolic *sy, u64 max_obj, const qd_params &prm, qd_step_stats &st) {
@@ -2067,18 +2270,56 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     // range step places it in the slab, a single pass in a buffer of its
     // own, and both fill it with a second prep launch.
     const u64 tab_bytes = (sm_tab_base(in_bytes) + kSmSlots * 64 + 16) * sizeof(u64);
-    bool defer_tab = KIND == QD_RULE_QCGD_SPLIT_MERGE && !BATCH && fast && ctx->slab.p != nullptr;
+    bool defer_tab =
+        KIND == QD_RULE_QCGD_SPLIT_MERGE && !BATCH && fast && ctx->slab.p != nullptr && N > 65536;  // (60 MB at most)
     if (ctx->tab.view) ctx->tab.release();  // a view into the slab is this step's to place again
     if (KIND == QD_RULE_QCGD_SPLIT_MERGE && !defer_tab) QD_TRY(ensure_relieved(ctx, ctx->tab, tab_bytes));
     u64 *counters = ctx->counters.as<u64>();
     // counters: [0] unique count, [1] select count A, [2] select count B,
     // [3] low: max child size, [4] low: error word, [5] oversized buckets
-    QD_HIP(hipMemsetAsync(counters, 0, 64 * sizeof(u64), s));
     u32 *maxsz = reinterpret_cast<u32 *>(counters + 3);
     u32 *errw = reinterpret_cast<u32 *>(counters + 4);
     if (BATCH && !fast) return fail(QD_ERR_UNSUPPORTED, "the batched step needs the QCGD fast path");
     u64 *hb = ctx->host;
+    // the rest of the step may be driven from the device: plain top-K keys,
+    // the default layout, no hook between the phases
+    bool lean = !BATCH && lean_allowed(ctx, sk) && max_obj != 0 && N <= kLeanMax && (KIND == QD_RULE_HADAMARD || fast);
+    // room for the candidates is made before their number is known when it
+    // follows from the parents' (hadamard), or when there are few parents (a
+    // wait for it costs more than launches that return at once); otherwise
+    // the host waits for it
+    u64 room = 0;
+    if (lean && KIND == QD_RULE_HADAMARD) room = 2 * N;
+    else if (lean && N <= kLeanSpecParents) room = kLeanSpec;
+    if (room > kLeanMax) room = 0;
+    // (what the caller lets one pass take; hadamard steps have one pass only)
+    const u64 lean_max = fast && ctx->tune.chunk_log2 ? std::min<u64>(kLeanMax, 1ull << ctx->tune.chunk_log2) : kLeanMax;
+    if (room > lean_max) room = 0;
+    const LeanArea la(N);
+    QD_TRY(ensure_relieved(ctx, ctx->lean, la.words * sizeof(u64)));
+    QD_TRY(ensure_relieved(ctx, ctx->ctab, kLeanTab * sizeof(u64)));
+    i32 *delta = nullptr;
+    if (lean && KIND == QD_RULE_QCGD_SPLIT_MERGE) {
+        QD_TRY(ensure_relieved(ctx, ctx->delta, (sm_delta_base(in_bytes) + 64) * sizeof(i32)));
+        delta = ctx->delta.as<i32>();
+    }
+    hipLaunchKernelGGL(k_lean_clear, dim3(grid_for(la.words, 256, 256)), dim3(256), 0, s, ctx->lean.as<u64>(), la.words,
+                       counters, u64(64));
     u64 nitems = 0;  // work items of the fast generate
+    const ScanReport *scan = reinterpret_cast<const ScanReport *>(ctx->host + kHostScan);
+    auto scan_parents = [&](const u32 *wi) -> int {
+        u64 *a = ctx->lean.as<u64>();
+        prof_begin(ctx, QD_PHASE_SCAN);
+        hipLaunchKernelGGL(k_lean_scan, dim3(unsigned(la.scan_tiles)), dim3(kScanThreads), 0, s,
+                           (const u32 *)ctx->nc.as<u32>(), wi, N, u32(la.scan_tiles), ctx->cb.as<u64>(),
+                           ctx->wb.as<u64>(), ctx->ctab.as<u64>(), kLeanTab, room ? room : kLeanMax,
+                           (const u32 *)maxsz, (const u32 *)errw, reinterpret_cast<LeanPlan *>(a), a + la.scan_desc,
+                           a + la.scan_desc + la.scan_tiles, reinterpret_cast<ScanReport *>(ctx->host + kHostScan));
+        QD_HIP(hipGetLastError());
+        prof_end(ctx, QD_PHASE_SCAN);
+        return QD_OK;
+    };
+    LeanEnd le;
     if (fast) {
         QD_TRY(ensure_relieved(ctx, ctx->pdesc, N * sizeof(PDesc)));
         QD_TRY(ensure_relieved(ctx, ctx->wi, N * sizeof(u32)));
@@ -2093,58 +2334,83 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
         prof_begin(ctx, QD_PHASE_PREP);
         hipLaunchKernelGGL(k_prep_fast<KIND>, dim3(grid_for(N, 16, 65536)), dim3(256), 0, s, P, keep,
                            ctx->pdesc.as<PDesc>(), ctx->nc.as<u32>(), ctx->wi.as<u32>(),
-                           defer_tab ? (u64 *)nullptr : ctx->tab.as<u64>(), maxsz, errw);
+                           defer_tab ? (u64 *)nullptr : ctx->tab.as<u64>(), delta, maxsz, errw);
         QD_HIP(hipGetLastError());
         prof_end(ctx, QD_PHASE_PREP);
-        prof_begin(ctx, QD_PHASE_SCAN);
-        QD_TRY(run_scan(ctx, LoadU32{ctx->nc.as<u32>()}, N, ctx->cb.as<u64>()));
-        QD_TRY(run_scan(ctx, LoadU32{ctx->wi.as<u32>()}, N, ctx->wb.as<u64>()));
-        prof_end(ctx, QD_PHASE_SCAN);
-        QD_HIP(hipMemcpyAsync(hb, ctx->cb.as<u64>() + N, sizeof(u64), hipMemcpyDeviceToHost, s));
-        QD_HIP(hipMemcpyAsync(hb + 1, counters + 3, 2 * sizeof(u64), hipMemcpyDeviceToHost, s));
-        QD_HIP(hipMemcpyAsync(hb + 3, ctx->wb.as<u64>() + N, sizeof(u64), hipMemcpyDeviceToHost, s));
-        QD_HIP(hipStreamSynchronize(s));
-        prof_collect(ctx);
-        nitems = hb[3];
-        if (nitems && !(u32(hb[2]) & ERR_WIDE)) {
-            const u64 nchunk = (nitems + kGenThreads - 1) / kGenThreads;
-            QD_TRY(ensure_relieved(ctx, ctx->cpar, nchunk * sizeof(u64)));
-            hipLaunchKernelGGL(k_chunk_parent, dim3(grid_for(nchunk)), dim3(256), 0, s, ctx->wb.as<u64>(), N, nchunk,
-                               ctx->cpar.as<u64>());
-            QD_HIP(hipGetLastError());
-        }
-        if (BATCH && (u32(hb[2]) & ERR_WIDE))
-            return fail(QD_ERR_UNSUPPORTED, "the batched step handles graphs of at most 64 nodes");
-        if (u32(hb[2]) & ERR_WIDE) {  // a graph wider than 64 nodes: generic kernels
-            fast = false;
-            QD_HIP(hipMemsetAsync(counters + 3, 0, 2 * sizeof(u64), s));
-            if (defer_tab) {  // the generic prep fills it
-                release_range_cache(ctx);
-                QD_TRY(ensure_relieved(ctx, ctx->tab, tab_bytes));
-                defer_tab = false;
-            }
-        }
-    }
-    if (!fast) {
+        QD_TRY(scan_parents(ctx->wi.as<u32>()));
+    } else {
         prof_begin(ctx, QD_PHASE_PREP);
         hipLaunchKernelGGL(k_prep<KIND>, dim3(grid_for(N)), dim3(256), 0, s, P, keep, rule, ctx->nc.as<u32>(),
                            ctx->pre.as<u64>(), ctx->tab.as<u64>(), maxsz, errw);
         QD_HIP(hipGetLastError());
         prof_end(ctx, QD_PHASE_PREP);
-        prof_begin(ctx, QD_PHASE_SCAN);
-        QD_TRY(run_scan(ctx, LoadU32{ctx->nc.as<u32>()}, N, ctx->cb.as<u64>()));
-        prof_end(ctx, QD_PHASE_SCAN);
-        QD_HIP(hipMemcpyAsync(hb, ctx->cb.as<u64>() + N, sizeof(u64), hipMemcpyDeviceToHost, s));
-        QD_HIP(hipMemcpyAsync(hb + 1, counters + 3, 2 * sizeof(u64), hipMemcpyDeviceToHost, s));
+        QD_TRY(scan_parents(nullptr));
+    }
+    if (room) {
+        QD_TRY(lean_tail<KIND>(ctx, P, rule, la, room, 0, 0, max_obj, prm, out, st, le));
+    } else {
         QD_HIP(hipStreamSynchronize(s));
         prof_collect(ctx);
     }
+    if (fast && (scan->err & ERR_WIDE)) {
+        if (BATCH) return fail(QD_ERR_UNSUPPORTED, "the batched step handles graphs of at most 64 nodes");
+        // a graph wider than 64 nodes: generic kernels
+        fast = lean = false;
+        hipLaunchKernelGGL(k_lean_clear, dim3(grid_for(la.words, 256, 256)), dim3(256), 0, s, ctx->lean.as<u64>(),
+                           la.words, counters + 3, u64(2));
+        if (defer_tab) {  // the generic prep fills it
+            release_range_cache(ctx);
+            QD_TRY(ensure_relieved(ctx, ctx->tab, tab_bytes));
+            defer_tab = false;
+        }
+        prof_begin(ctx, QD_PHASE_PREP);
+        hipLaunchKernelGGL(k_prep<KIND>, dim3(grid_for(N)), dim3(256), 0, s, P, keep, rule, ctx->nc.as<u32>(),
+                           ctx->pre.as<u64>(), ctx->tab.as<u64>(), maxsz, errw);
+        QD_HIP(hipGetLastError());
+        prof_end(ctx, QD_PHASE_PREP);
+        QD_TRY(scan_parents(nullptr));
+        QD_HIP(hipStreamSynchronize(s));
+        prof_collect(ctx);
+    }
+    nitems = scan->items;
+    hb[0] = scan->C;
+    hb[1] = scan->maxsz;
+    hb[2] = scan->err;
     const u64 C = hb[0];
     const u32 max_child = u32(hb[1]);  // largest child size (bytes) of the kept parents
     QD_TRY(check_err_word(u32(hb[2])));
     st.num_candidates = C;
     if (BATCH) QD_TRY(batch_cseg(ctx, bt));
     if (C == 0) return finish_empty();
+    if (lean && !le.done && C <= lean_max && !(le.stop & ~LEAN_BIG)) {
+        if (defer_tab) {
+            QD_TRY(ensure_relieved(ctx, ctx->tab, tab_bytes));
+            hipLaunchKernelGGL(k_prep_fast<KIND>, dim3(grid_for(N, 16, 65536)), dim3(256), 0, s, P, keep,
+                               ctx->pdesc.as<PDesc>(), ctx->nc.as<u32>(), ctx->wi.as<u32>(), ctx->tab.as<u64>(), delta,
+                               maxsz, errw);
+            QD_HIP(hipGetLastError());
+            defer_tab = false;
+        }
+        QD_TRY(lean_tail<KIND>(ctx, P, rule, la, C, C, nitems, max_obj, prm, out, st, le));
+    }
+    if (le.done) {
+        u32 b1, b2;
+        dedup_layout(C, ctx->tune, b1, b2);
+        st.dedup_levels = (b1 ? 1 : 0) + (b2 ? 1 : 0);
+        if (st.num_survivors == 0) return finish_empty();
+        if (sy) {
+            sy->num_object = C;
+            sy->num_object_after_interferences = st.num_unique;
+        }
+        return QD_OK;
+    }
+    if (fast && nitems) {
+        const u64 nchunk = (nitems + kGenThreads - 1) / kGenThreads;
+        QD_TRY(ensure_relieved(ctx, ctx->cpar, nchunk * sizeof(u64)));
+        hipLaunchKernelGGL(k_chunk_parent, dim3(grid_for(nchunk)), dim3(256), 0, s, ctx->wb.as<u64>(), N, nchunk,
+                           ctx->cpar.as<u64>());
+        QD_HIP(hipGetLastError());
+    }
     if (!BATCH && fast) {
         const u64 budget = step_budget(ctx);
         if (C > budget) {
@@ -2168,8 +2434,8 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
         QD_TRY(ensure_relieved(ctx, ctx->tab, tab_bytes));
         prof_begin(ctx, QD_PHASE_PREP);
         hipLaunchKernelGGL(k_prep_fast<KIND>, dim3(grid_for(N, 16, 65536)), dim3(256), 0, s, P, keep,
-                           ctx->pdesc.as<PDesc>(), ctx->nc.as<u32>(), ctx->wi.as<u32>(), ctx->tab.as<u64>(), maxsz,
-                           errw);
+                           ctx->pdesc.as<PDesc>(), ctx->nc.as<u32>(), ctx->wi.as<u32>(), ctx->tab.as<u64>(),
+                           (i32 *)nullptr, maxsz, errw);
         QD_HIP(hipGetLastError());
         prof_end(ctx, QD_PHASE_PREP);
     }
@@ -2209,7 +2475,11 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     QD_HIP(hipMemsetAsync(ctx->nhist.p, 0, kHistBins * sizeof(u64), s));
     phase_mark(ctx, PH_SYMBOLIC);
     u64 in_stride = 0;
-    if (fused) {
+    // (a device-driven step that stopped in the select is taken up after the
+    // dedup: its uniques are in place)
+    const bool deduped = le.stop == LEAN_SELECT;
+    if (deduped) fused = true;
+    if (fused && !deduped) {
         const unsigned gg =
             unsigned(std::min<u64>((nitems + kGenThreads - 1) / kGenThreads, ctx->tune.generate_grid));
         QD_HIP(hipMemsetAsync(ctx->cur1.p, 0, nbin1 * sizeof(u64), s));
@@ -2265,7 +2535,16 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     double2 *UM;
     u64 U;
     phase_mark(ctx, PH_COLL_PREP);
-    QD_TRY(partition_dedup(ctx, H0, M0, nullptr, C, b1, b2, prm.tolerance, st, UH, UR, UM, U, in_stride, UK));
+    if (deduped) {
+        UH = H0;
+        UR = UH + C;
+        UM = reinterpret_cast<double2 *>(UR + C);
+        U = le.U;
+        QD_HIP(hipMemcpyAsync(ctx->nhist.p, ctx->lean.as<u64>() + la.nhist, kHistBins * sizeof(u64),
+                              hipMemcpyDeviceToDevice, s));
+    } else {
+        QD_TRY(partition_dedup(ctx, H0, M0, nullptr, C, b1, b2, prm.tolerance, st, UH, UR, UM, U, in_stride, UK));
+    }
     phase_mark(ctx, PH_COLL_FINAL);
     st.num_unique = U;
 
@@ -2626,8 +2905,8 @@ static int adjoint_kind(qd_ctx *ctx, qd_state *in, const qd_rule &rule, const qd
         QD_TRY(ctx->wi.ensure(N * sizeof(u32)));
         QD_TRY(ctx->wb.ensure((N + 1) * sizeof(u64)));
         hipLaunchKernelGGL(k_prep_fast<KIND>, dim3(grid_for(N, 16, 65536)), dim3(256), 0, s, P, (const u64 *)nullptr,
-                           ctx->pdesc.as<PDesc>(), ctx->nc.as<u32>(), ctx->wi.as<u32>(), ctx->tab.as<u64>(), maxsz,
-                           errw);
+                           ctx->pdesc.as<PDesc>(), ctx->nc.as<u32>(), ctx->wi.as<u32>(), ctx->tab.as<u64>(),
+                           (i32 *)nullptr, maxsz, errw);
         QD_HIP(hipGetLastError());
         QD_TRY(run_scan(ctx, LoadU32{ctx->nc.as<u32>()}, N, ctx->cb.as<u64>()));
         QD_TRY(run_scan(ctx, LoadU32{ctx->wi.as<u32>()}, N, ctx->wb.as<u64>()));

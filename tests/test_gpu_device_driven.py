@@ -1,0 +1,112 @@
+"""The step driven from the device (qd_k_lean.hpp) at the edges of its tiles,
+bucket layouts and rooms, bit for bit against the oracle, and against the
+host-driven path (qd_tuning.eager_select) where the oracle would take long."""
+import math
+
+import numpy as np
+import pytest
+
+import quids_amd as q
+from oracle import oracle as orc
+from quids_amd.rules import qcgd
+from quids_amd.rules import quantum_computer as qc
+from quids_amd.state import HostState
+
+from helpers import assert_states_identical, qcgd_initial
+
+pytestmark = pytest.mark.gpu
+
+
+def _registers(n, equal=False):
+    """n distinct registers of 4 bytes: the qubit that the gate acts on and a
+    number of 20 bits; random or equal magnitudes."""
+    rng = np.random.default_rng(n)
+    v = rng.permutation(1 << 20)[:n].astype(np.uint32)
+    obj = np.zeros((n, 8), np.uint8)
+    for k in range(3):
+        obj[:, 1 + k] = (v >> (8 * k)) & 0xFF
+    obj[:, 0] = rng.integers(0, 2, n)  # the qubit the gate acts on
+    mag = rng.normal(size=n) + 1j * rng.normal(size=n)
+    if equal:
+        mag = np.full(n, 1 + 0j)
+    return HostState(obj.reshape(-1), np.arange(n + 1, dtype=np.uint64) * np.uint64(8), np.full(n, 4, np.uint32),
+                     mag / np.linalg.norm(mag))
+
+
+def _step(hs, rule, cap, **tuning):
+    ctx = q.default_context()
+    old = ctx.get_tuning()
+    ctx.set_tuning(**tuning)
+    try:
+        a, b = q.it_t(), q.it_t()
+        a.upload(hs)
+        out = []
+        for _ in range(2):  # a fresh output state, then one that has room
+            st = q.simulate(a, rule, b, None, cap)
+            out.append(b.download())
+        assert_states_identical(out[0], out[1], "repeated")
+        return out[1], st
+    finally:
+        ctx.set_tuning(**{k: old[k] for k in tuning})
+
+
+# candidates 2n: around the generate's chunk (1024), the order's tile (4096),
+# the bucket layouts (128 per bucket, one pass of 480 x 256, the sub-buckets)
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 512, 513, 2047, 2048, 2049, 16384, 16385, 61440, 61441, 140000])
+def test_hadamard_sizes(n):
+    hs = _registers(n)
+    for cap in (q.UINT64_MAX, 2 * n, max(1, n + n // 3), max(1, n)):
+        g, st = _step(hs, qc.hadamard(0), cap)
+        o, ost = orc.simulate(hs, qc.hadamard(0), cap)
+        assert (st["num_candidates"], st["num_unique"]) == (2 * n, ost["num_unique"])
+        assert_states_identical(g, o, f"n {n} cap {cap}")
+
+
+# as many equal |m|^2 as the finishing block takes, one more, and many
+@pytest.mark.parametrize("n", [100, 4096, 4097, 30000])
+def test_equal_magnitudes(n):
+    hs = _registers(n, equal=True)
+    for cap in (n, n + n // 2):
+        g, _ = _step(hs, qc.hadamard(0), cap)
+        o, _ = orc.simulate(hs, qc.hadamard(0), cap)
+        assert_states_identical(g, o, f"equal {n} cap {cap}")
+
+
+# parents around the number up to which the host does not wait for the
+# candidates' number, with few candidates, and more than it made room for
+@pytest.mark.parametrize("parents", [40, 2047, 2048, 2049])
+@pytest.mark.parametrize("nodes", [7, 11])
+@pytest.mark.parametrize("rule", [qcgd.split_merge(0.8, 0.3), qcgd.erase_create(1.1, 0.5), qcgd.coin(0.9, 0.2)])
+def test_qcgd_parents(parents, nodes, rule):
+    hs = qcgd_initial(nodes, 42)
+    for r in (qcgd.split_merge(0.7, 0.2), qcgd.erase_create(1.0, 0.4)) * 2:
+        hs = orc.simulate(hs, r, parents)[0]
+        hs = orc.apply_modifier(hs, qcgd.step)
+    for cap in (max(hs.num_object, 1000), q.UINT64_MAX):
+        if cap == q.UINT64_MAX and nodes == 11 and parents > 40:
+            continue
+        g, st = _step(hs, rule, cap)
+        o, ost = orc.simulate(hs, rule, cap)
+        assert (st["num_candidates"], st["num_unique"]) == (ost["num_candidates"], ost["num_unique"])
+        assert_states_identical(g, o, f"{type(rule).__name__} {parents} cap {cap}")
+
+
+# 0.7e6 to 2e7 candidates: one child per lane, by work items, and beyond what
+# the device drives
+@pytest.mark.parametrize("parents", [9000, 60000, 150000])
+def test_large_steps_match_the_host_driven_path(parents):
+    a, b = q.it_t(), q.it_t()
+    a.upload(HostState.from_objects([qcgd.seeded_graph(12, 42)]))
+    rules = [qcgd.split_merge(math.pi / 4, 0.1), qcgd.erase_create(math.pi / 3, math.pi / 5)]
+    for k in range(5):
+        if k % 2 == 0:
+            q.simulate(a, qcgd.step)
+        q.simulate(a, rules[k % 2], b, None, parents // 4 if k < 4 else parents)
+        a, b = b, a
+    hs = a.download()
+    got = {}
+    for eager in (0, 1):
+        for i, r in enumerate(rules):
+            got[eager, i], _ = _step(hs, r, parents, eager_select=eager)
+    for i in range(2):
+        assert_states_identical(got[0, i], got[1, i], f"{parents} rule {i}")
