@@ -93,8 +93,8 @@ static_assert(LEAN_SPILL == ERR_SPILL1, "the work items' generate reports its sp
 
 // Buckets of C candidates: while one radix pass of at most 2^8 buckets is
 // enough, buckets of at most 128 (their dedup blocks all run at once), then
-// of at most 480 entries on average, in a capacity of at most 1024 (the
-// dedup table): 16 sigma and 256 entries beyond the mean, as sub-buckets
+// of at most 480 entries on average, in a capacity of at most 1000 (the
+// dedup table holds 1024): 16 sigma and 256 entries beyond the mean, as sub-buckets
 // whose hashes repeat spread more than distinct ones.
 QD_HD void lean_layout(u64 C, u32 &b1, u32 &b2, u64 &cap1, u64 &cap2) {
     u32 L = 0;
@@ -108,9 +108,9 @@ QD_HD void lean_layout(u64 C, u32 &b1, u32 &b2, u64 &cap1, u64 &cap2) {
         return 16 * r;
     };
     const u64 m1 = (C >> b1) + 1, m2 = (C >> L) + 1;
-    cap1 = b2 ? m1 + slack(m1) + 4096 : 1024;
+    cap1 = b2 ? m1 + slack(m1) + 4096 : 1000;
     cap2 = b2 ? (m2 + slack(m2) + 256 + 63) / 64 * 64 : 0;
-    if (cap2 > 1024) cap2 = 1024;
+    if (cap2 > 1000) cap2 = 1000;
 }
 
 // Reports of the scan to the host (pinned memory).

@@ -858,15 +858,23 @@ static int partition_dedup(qd_ctx *ctx, const u64 *H0, const double2 *M0, const 
     } else {
         const u64 nb = 1ull << (b1 + b2);
         const u64 mean = (n + nb - 1) / nb;
-        // mean + 6 sigma + 128 (sub-bucket sizes are near Poisson; a spill
-        // takes the exact path)
-        const u64 cap2 = (mean + u64(6.0 * std::sqrt(double(mean))) + 128 + 63) / 64 * 64;
+        // mean + 16 sigma + 256, at most about what the dedup's table takes,
+        // where the pass budget's buffer holds that (hashes that repeat, as
+        // split_merge's do, spread the sub-buckets more than distinct ones:
+        // at 6 sigma a 12-node step of 1.7e8 candidates spilled and paid a
+        // second, exact pass of 5.5 ms), else mean + 6 sigma + 128; a spill
+        // takes the exact path.  (A stride of 1016 entries made the pass 10 %
+        // slower; 768 to 1000 and 1024 read the same.)
+        const u64 sg6 = u64(6.0 * std::sqrt(double(mean))), sg16 = u64(16.0 * std::sqrt(double(mean)));
+        const u64 full2 = u64(double(step_budget(ctx)) * 1.8);
+        u64 cap2 = (mean + sg6 + 128 + 63) / 64 * 64;
+        const u64 wide2 = std::min<u64>((mean + sg16 + 256 + 63) / 64 * 64, ctx->tune.dedup_cap - 24);
+        if (wide2 > cap2 && nb * wide2 <= std::max<u64>(full2, n)) cap2 = wide2;
         QD_TRY(ctx->off2.ensure((nb + 1) * sizeof(u64)));
         QD_TRY(ctx->cnt2.ensure(nb * sizeof(u64)));
         // fixed-capacity sub-buckets unless their padding would pass the
         // pass budget's buffer (small sub-buckets near the budget): then
         // exact offsets from a counting pass
-        const u64 full2 = u64(double(step_budget(ctx)) * 1.8);
         const bool fixed = nb * cap2 <= std::max<u64>(full2, n);
         QD_TRY(ensure_big(ctx->ebuf2, std::max<u64>(fixed ? nb * cap2 : n, n) * sizeof(Entry), full2 * sizeof(Entry)));
         Entry *E2 = ctx->ebuf2.as<Entry>();
