@@ -923,7 +923,7 @@ static int partition_dedup(qd_ctx *ctx, const u64 *H0, const double2 *M0, const 
 // Regenerates the K survivors (candidate indices orep, ascending; their
 // magnitudes already in out->mag) into out: sizes, padded offsets, bytes.
 template <int KIND>
-static int populate_out(qd_ctx *ctx, const Parents &P, const qd_rule &rule, const u64 *orep, u64 K,
+static int populate_out(qd_ctx *ctx, const Parents &P, const PDesc *D, const qd_rule &rule, const u64 *orep, u64 K,
                         const qd_params &prm, qd_state *out, qd_step_stats &st) {
     hipStream_t s = ctx->stream;
     u64 *hb = ctx->host;
@@ -940,16 +940,15 @@ static int populate_out(qd_ctx *ctx, const Parents &P, const qd_rule &rule, cons
     // the state's if the state needs it)
     QD_TRY(ensure_relieved(ctx, out->objects, std::max<u64>(bytes, 1)));
     prof_begin(ctx, QD_PHASE_FINALIZE);
+    const unsigned gp = unsigned(std::min<u64>((K + 3) / 4, 65536));
     if (KIND == QD_RULE_QCGD_SPLIT_MERGE)
-        hipLaunchKernelGGL(k_populate_sm, dim3(unsigned(std::min<u64>((K + kPopSegs - 1) / kPopSegs, 65536))),
-                           dim3(kWave), 0, s, P,
-                           ctx->cb.as<u64>(), rule, orep, (const u64 *)ctx->opar.as<u64>(), K, out->begin.as<u64>(),
-                           out->size.as<u32>(), out->objects.as<u8>(), (const LeanPlan *)nullptr, u64(0));
+        hipLaunchKernelGGL(k_populate_sm, dim3(gp), dim3(kWave), 0, s, P, (const u64 *)ctx->cb.as<u64>(), orep,
+                           (const u64 *)ctx->opar.as<u64>(), K, (const u64 *)out->begin.as<u64>(),
+                           out->objects.as<u8>(), (const LeanPlan *)nullptr, u64(0));
     else
-        hipLaunchKernelGGL(k_populate_flip<KIND>, dim3(unsigned(std::min<u64>((K + 7) / 8, 65536))), dim3(256), 0, s,
-                           P, ctx->cb.as<u64>(), rule, orep, (const u64 *)ctx->opar.as<u64>(), K,
-                           out->begin.as<u64>(), out->size.as<u32>(), out->objects.as<u8>(),
-                           (const LeanPlan *)nullptr, u64(0));
+        hipLaunchKernelGGL(k_populate_flip<KIND>, dim3(gp), dim3(kWave), 0, s, P, D, (const u64 *)ctx->cb.as<u64>(),
+                           rule, orep, (const u64 *)ctx->opar.as<u64>(), K, (const u64 *)out->begin.as<u64>(),
+                           out->objects.as<u8>(), (const LeanPlan *)nullptr, u64(0));
     QD_HIP(hipGetLastError());
     out->n = K;
     out->bytes = bytes;
@@ -1786,7 +1785,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
     QD_HIP(hipGetLastError());
     prof_end(ctx, QD_PHASE_ORDER);
     phase_mark(ctx, PH_FINAL);
-    QD_TRY(populate_out<KIND>(ctx, P, rule, orep, K, prm, out, st));
+    QD_TRY(populate_out<KIND>(ctx, P, ctx->pdesc.as<PDesc>(), rule, orep, K, prm, out, st));
     phase_mark(ctx, PH_NORMALIZE);
     QD_TRY(normalize_state(ctx, out));
     prof_collect(ctx);
@@ -2162,14 +2161,13 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, const qd_rule &rule, const L
         prof_end(ctx, QD_PHASE_ORDER);
         prof_begin(ctx, QD_PHASE_FINALIZE);
         if (KIND == QD_RULE_QCGD_SPLIT_MERGE)
-            hipLaunchKernelGGL(k_populate_sm, dim3(grid_for(bound, kPopSegs, 8192)), dim3(kWave), 0, s, P, cb, rule,
+            hipLaunchKernelGGL(k_populate_sm, dim3(grid_for(bound, 4, 16384)), dim3(kWave), 0, s, P, cb,
                                (const u64 *)ctx->keys.as<u64>(), (const u64 *)ctx->opar.as<u64>(), capk,
-                               (const u64 *)out->begin.as<u64>(), (const u32 *)out->size.as<u32>(),
-                               out->objects.as<u8>(), (const LeanPlan *)lp, capb);
+                               (const u64 *)out->begin.as<u64>(), out->objects.as<u8>(), (const LeanPlan *)lp, capb);
         else
-            hipLaunchKernelGGL(k_populate_flip<KIND>, dim3(grid_for(bound, 8, 8192)), dim3(256), 0, s, P, cb, rule,
-                               (const u64 *)ctx->keys.as<u64>(), (const u64 *)ctx->opar.as<u64>(), capk,
-                               (const u64 *)out->begin.as<u64>(), (const u32 *)out->size.as<u32>(),
+            hipLaunchKernelGGL(k_populate_flip<KIND>, dim3(grid_for(bound, 8, 16384)), dim3(kWave), 0, s, P,
+                               (const PDesc *)ctx->pdesc.as<PDesc>(), cb, rule, (const u64 *)ctx->keys.as<u64>(),
+                               (const u64 *)ctx->opar.as<u64>(), capk, (const u64 *)out->begin.as<u64>(),
                                out->objects.as<u8>(), (const LeanPlan *)lp, capb);
         QD_HIP(hipGetLastError());
         prof_end(ctx, QD_PHASE_FINALIZE);
@@ -2595,7 +2593,7 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
                        ctx->wprefix.as<u64>(), orep, out->mag.as<double2>());
     prof_end(ctx, QD_PHASE_ORDER);
     phase_mark(ctx, PH_FINAL);
-    QD_TRY(populate_out<KIND>(ctx, P, rule, orep, K, prm, out, st));
+    QD_TRY(populate_out<KIND>(ctx, P, fast ? ctx->pdesc.as<PDesc>() : nullptr, rule, orep, K, prm, out, st));
     // ---- 9 normalize
     phase_mark(ctx, PH_NORMALIZE);
     if (BATCH) QD_TRY(batch_normalize(ctx, bt, out));

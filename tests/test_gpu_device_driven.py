@@ -12,7 +12,7 @@ from quids_amd.rules import qcgd
 from quids_amd.rules import quantum_computer as qc
 from quids_amd.state import HostState
 
-from helpers import assert_states_identical, qcgd_initial
+from helpers import assert_states_identical, qcgd_initial, sparse_graph
 
 pytestmark = pytest.mark.gpu
 
@@ -110,3 +110,39 @@ def test_large_steps_match_the_host_driven_path(parents):
             got[eager, i], _ = _step(hs, r, parents, eager_select=eager)
     for i in range(2):
         assert_states_identical(got[0, i], got[1, i], f"{parents} rule {i}")
+
+
+# survivors' bytes: graphs around the lane segments' widths (16, 32, 64 nodes;
+# beyond, the whole step runs on the generic kernels), children beyond the
+# lists of 64 nodes and 128 names, at every alignment
+@pytest.mark.parametrize("align", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("nodes", [(1, 2), (15, 16), (16, 17), (31, 32, 33), (60, 63, 64), (64, 65)])
+def test_populate_widths(nodes, align):
+    old = q.align_byte_length
+    q.align_byte_length = align
+    try:
+        objs = []
+        for n in nodes:
+            objs.append(sparse_graph(n, tuple(range(0, n, max(n // 5, 1))), ()))
+            objs.append(sparse_graph(n, (n // 2,), (n // 3,) if n > 3 else ()))
+        hs = HostState.from_objects(objs, align=align)
+        for k, r in enumerate((qcgd.split_merge(0.8, 0.3), qcgd.coin(0.9, 0.2)) * 3):
+            a, b = q.it_t(), q.it_t()
+            a.upload(hs)
+            q.simulate(a, r, b, None, 3000)
+            ref, _ = orc.simulate(hs, r, 3000, align=align)
+            assert_states_identical(b.download(), ref, f"{nodes} align {align} step {k}")
+            hs = orc.apply_modifier(ref, qcgd.step)
+    finally:
+        q.align_byte_length = old
+
+
+@pytest.mark.parametrize("size", [1, 3, 8, 9, 17, 64, 200])
+def test_populate_register_sizes(size):
+    rng = np.random.default_rng(size)
+    objs = {bytes(rng.integers(0, 2, size).astype(np.uint8)) for _ in range(300)}
+    hs = HostState.from_objects(sorted(objs))
+    for bit in {0, size // 2, size - 1}:
+        g, _ = _step(hs, qc.hadamard(bit), q.UINT64_MAX)
+        o, _ = orc.simulate(hs, qc.hadamard(bit))
+        assert_states_identical(g, o, f"size {size} bit {bit}")
