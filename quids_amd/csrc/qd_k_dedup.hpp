@@ -399,13 +399,15 @@ __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const 
     if (threadIdx.x == 0) ocount = 0;
     u64 uniques = 0;  // thread 0's running total
 
+    // (entries beyond a fixed capacity lie in the overflow list)
+    const u64 lim = rstride && rstride < u64(CAP) ? rstride : u64(CAP);
     Entry x[PER];
     u64 nbeg = 0, nnum = 0;
     auto fetch = [&](u64 bb) {
         nbeg = woff[bb];
         nnum = woff[bb + 1] - nbeg;
         const u64 rb = rstride ? bb * rstride : nbeg;
-        if (nnum <= CAP) {
+        if (nnum <= lim) {
 #pragma unroll
             for (int k = 0; k < PER; ++k) {
                 const u32 i = threadIdx.x + T * k;
@@ -417,7 +419,7 @@ __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const 
     __syncthreads();
     for (u64 b = blockIdx.x; b < nbk; b += gridDim.x) {
         const u64 beg = nbeg, nn = nnum;  // uniform over the block
-        if (nn > CAP) {
+        if (nn > lim) {
             if (threadIdx.x == 0) biglist[atomicAdd(reinterpret_cast<unsigned long long *>(counters + 5), 1ull)] = b;
             __syncthreads();
             if (b + gridDim.x < nbk) fetch(b + gridDim.x);
@@ -679,35 +681,51 @@ __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const 
     if (threadIdx.x == 0 && uniques) atomicAdd(reinterpret_cast<unsigned long long *>(counters), uniques);
 }
 
-// The same computation for buckets beyond the LDS capacity, one workgroup
-// per bucket, on a global scratch region (rare: a bucket this large needs a
-// group of thousands of candidates with one hash).  Scratch of listed bucket
-// q starts at soff[q] elements: keys, cands, mags (npad each) and u32 segs.
-__global__ __launch_bounds__(1024) void k_dedup_big(const Entry *E, u64 rstride, const u64 *boff, const u64 *biglist,
-                                                    const u64 *soff, u64 *skeyg, u64 *scandg, double2 *smagg,
-                                                    u32 *segg, double tol, u64 *UH, u64 *UR, double2 *UM,
-                                                    u32 *UK, u64 *counters, u64 *nhist) {
-    __shared__ u32 maxg;
+// The same computation for buckets beyond the LDS capacity or their fixed
+// one, one workgroup per bucket, on a global scratch region (rare: such a
+// bucket needs a group of hundreds of candidates with one hash).  Bucket b's
+// entries are the first min(count, rstride) of its range and those of the
+// overflow list whose top L hash bits are b (modulo the nbk buckets).
+// Scratch of listed bucket q starts at soff[q] elements: keys, cands, mags
+// (npad each) and u32 segs.
+__global__ __launch_bounds__(1024) void k_dedup_big(const Entry *E, u64 rstride, const Entry *ovf, u64 novf, u32 L,
+                                                    u64 nbk, const u64 *boff, const u64 *biglist, const u64 *soff,
+                                                    u64 *skeyg, u64 *scandg, double2 *smagg, u32 *segg, double tol,
+                                                    u64 *UH, u64 *UR, double2 *UM, u32 *UK, u64 *counters, u64 *nhist) {
+    __shared__ u32 maxg, fill;
     __shared__ u64 tmp[1024 / kWave + 1];
     const u64 b = biglist[blockIdx.x];
     const u64 beg = boff[b], n = boff[b + 1] - beg;
     const Entry *src = E + (rstride ? b * rstride : beg);
+    const u64 nsrc = rstride ? min(n, rstride) : n;
     u64 *skey = skeyg + soff[blockIdx.x];
     u64 *scand = scandg + soff[blockIdx.x];
     double2 *smag = smagg + soff[blockIdx.x];
     u32 *seg = segg + soff[blockIdx.x];
+    auto overflowed = [&](u64 h) { return ((L ? h >> (64 - L) : 0ull) & (nbk - 1)) == b; };
     u64 npad = 2;
     while (npad < n) npad <<= 1;
-    for (u64 i = threadIdx.x; i < npad; i += blockDim.x) {
-        if (i < n) {
-            skey[i] = src[i].hash;
-            scand[i] = src[i].cand;
-        } else {
-            skey[i] = ~0ull;
-            scand[i] = ~0ull;
-        }
+    if (threadIdx.x == 0) {
+        maxg = 1;
+        fill = u32(nsrc);
     }
-    if (threadIdx.x == 0) maxg = 1;
+    __syncthreads();
+    for (u64 i = threadIdx.x; i < nsrc; i += blockDim.x) {
+        skey[i] = src[i].hash;
+        scand[i] = src[i].cand;
+    }
+    if (nsrc < n)
+        for (u64 i = threadIdx.x; i < novf; i += blockDim.x) {
+            const u64 h = ovf[i].hash;
+            if (!overflowed(h)) continue;
+            const u32 at = atomicAdd(&fill, 1u);
+            skey[at] = h;
+            scand[at] = ovf[i].cand;
+        }
+    for (u64 i = n + threadIdx.x; i < npad; i += blockDim.x) {
+        skey[i] = ~0ull;
+        scand[i] = ~0ull;
+    }
     __syncthreads();
     for (u64 k = 2; k <= npad; k <<= 1) {
         for (u64 j = k >> 1; j > 0; j >>= 1) {
@@ -725,29 +743,39 @@ __global__ __launch_bounds__(1024) void k_dedup_big(const Entry *E, u64 rstride,
             __syncthreads();
         }
     }
-    // magnitudes: candidate c of this bucket is found by its position in the
-    // input (entries carry their candidate index, not their position), so
-    // re-read them by a search over the sorted (hash, cand) pairs
-    for (u64 i = threadIdx.x; i < n; i += blockDim.x) {
-        const u64 eh = src[i].hash, ec = src[i].cand;
+    // magnitudes: an entry's place is found by a search over the sorted
+    // (hash, cand) pairs
+    auto place = [&](const Entry &e) {
         u64 lo = 0, hi = n - 1;
         while (lo < hi) {
             const u64 mid = (lo + hi) >> 1;
-            if (key_gt(eh, ec, skey[mid], scand[mid])) lo = mid + 1;
+            if (key_gt(e.hash, e.cand, skey[mid], scand[mid])) lo = mid + 1;
             else hi = mid;
         }
-        smag[lo] = make_double2(src[i].re, src[i].im);
-    }
+        smag[lo] = make_double2(e.re, e.im);
+    };
+    for (u64 i = threadIdx.x; i < nsrc; i += blockDim.x) place(src[i]);
+    if (nsrc < n)
+        for (u64 i = threadIdx.x; i < novf; i += blockDim.x)
+            if (overflowed(ovf[i].hash)) place(ovf[i]);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        u32 run = 0;
-        for (u64 i = 0; i < n; ++i) {
-            if (i == 0 || skey[i] != skey[i - 1]) run = u32(i);
+    // each place's group start: a running maximum over the starts, a tile of
+    // the block's width at a time
+    u32 carry = 0;
+    for (u64 t0 = 0; t0 < n; t0 += blockDim.x) {
+        const u64 i = t0 + threadIdx.x;
+        const bool start = i < n && (i == 0 || skey[i] != skey[i - 1]);
+        const u32 here = start ? u32(i) : 0u;
+        const u32 run = max(max(block_excl_max(here, tmp), here), carry);
+        if (i < n) {
             seg[i] = run;
-            if (i + 1 - run > maxg) maxg = u32(i + 1 - run);
+            atomicMax(&maxg, u32(i) + 1 - run);
         }
+        if (threadIdx.x == blockDim.x - 1) tmp[0] = run;
+        __syncthreads();
+        carry = u32(tmp[0]);
+        __syncthreads();
     }
-    __syncthreads();
     for (u64 st = 1; st < maxg; st <<= 1) {
         for (u64 i = threadIdx.x; i < n; i += blockDim.x) {
             const u64 r = i - seg[i];
@@ -758,30 +786,39 @@ __global__ __launch_bounds__(1024) void k_dedup_big(const Entry *E, u64 rstride,
         }
         __syncthreads();
     }
-    // serial compaction by thread 0 (this path is rare)
-    if (threadIdx.x == 0) {
-        u64 pos = beg;
-        for (u64 i = 0; i < n; ++i) {
-            if (seg[i] != i) continue;
-            const double2 a = smag[i];
-            const double nrm = a.x * a.x + a.y * a.y;
-            if (nrm > tol) {
-                UH[pos] = skey[i];
-                UR[pos] = scand[i];
-                UM[pos] = a;
-                if (UK) UK[pos] = norm_top32(nrm);
-                ++pos;
-                atomicAdd(reinterpret_cast<unsigned long long *>(nhist + min(norm_top12(nrm), u32(kNormBins - 1))),
-                          1ull);
-            }
+    u64 pos = beg;
+    for (u64 t0 = 0; t0 < n; t0 += blockDim.x) {
+        const u64 i = t0 + threadIdx.x;
+        bool keep = false;
+        double nrm = 0.0;
+        double2 a = make_double2(0.0, 0.0);
+        if (i < n && seg[i] == i) {
+            a = smag[i];
+            nrm = a.x * a.x + a.y * a.y;
+            keep = nrm > tol;
         }
-        atomicAdd(reinterpret_cast<unsigned long long *>(counters), (unsigned long long)(pos - beg));
-        for (u64 j = pos; j < beg + n; ++j) {
-            UR[j] = kNoRep;
-            if (UK) UK[j] = 0;
+        u64 total;
+        const u64 at = pos + block_excl_scan(keep ? 1 : 0, tmp, total);
+        if (keep) {
+            UH[at] = skey[i];
+            UR[at] = scand[i];
+            UM[at] = a;
+            if (UK) UK[at] = norm_top32(nrm);
+            atomicAdd(reinterpret_cast<unsigned long long *>(nhist + min(norm_top12(nrm), u32(kNormBins - 1))), 1ull);
         }
+        pos += total;
+    }
+    if (threadIdx.x == 0) atomicAdd(reinterpret_cast<unsigned long long *>(counters), (unsigned long long)(pos - beg));
+    for (u64 j = pos + threadIdx.x; j < beg + n; j += blockDim.x) {
+        UR[j] = kNoRep;
+        if (UK) UK[j] = 0;
     }
 }
 
+// Counts of the listed buckets.
+__global__ __launch_bounds__(256) void k_big_counts(const u64 *boff, const u64 *biglist, u64 nbig, u64 *out) {
+    for (u64 q = u64(blockIdx.x) * blockDim.x + threadIdx.x; q < nbig; q += u64(gridDim.x) * blockDim.x)
+        out[q] = boff[biglist[q] + 1] - boff[biglist[q]];
+}
 
 }  // namespace qd

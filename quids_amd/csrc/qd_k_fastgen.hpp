@@ -1149,8 +1149,7 @@ __global__ __launch_bounds__(kGenThreads) void k_range_binwrite(const PDesc *D, 
 // pass again the two-walk way).  The block also counts its children per
 // first-level bucket (the top b1 key bits) as row blockIdx.x of bmat, so
 // that each group's regions merge into its first-level buckets at exact
-// offsets (k_range_colscan over the group's columns, k_excl_small,
-// k_region_place).
+// offsets (k_range_colscan, k_region_place).
 // ---------------------------------------------------------------------------
 constexpr u32 kRangeGroupsMax = 8;
 
@@ -1214,21 +1213,10 @@ __global__ __launch_bounds__(kGenThreads, kRangeWalkWaves<KIND>) void k_range_wa
     if (spill) atomicOr(err, ERR_SPILL1);
 }
 
-// off[i] = total[0] + ... + total[i - 1] for i <= n (n small).
-__global__ void k_excl_small(const u64 *total, u32 n, u64 *off) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        u64 acc = 0;
-        for (u32 i = 0; i < n; ++i) {
-            off[i] = acc;
-            acc += total[i];
-        }
-        off[n] = acc;
-    }
-}
-
 // Each region's entries at its running places in the buckets: bucket d
-// starts at boff[d], region r's first place in it is bm[r * bstride + d]
-// after the column scan.  A chunk of kPlaceChunk entries is ordered by bucket in LDS
+// holds total[d] entries (every block scans the nbin totals, and the first
+// writes the nbin + 1 offsets to off), region r's first place in it is
+// bm[r * bstride + d] after the column scan.  A chunk of kPlaceChunk entries is ordered by bucket in LDS
 // first, so that consecutive lanes write consecutive places of a bucket
 // (runs of about kPlaceChunk / nbin entries) rather than one entry to each
 // of up to 64 buckets per store.
@@ -1238,20 +1226,28 @@ constexpr u32 kPlaceChunk = kPlaceThreads * kPlacePer;
 
 __global__ __launch_bounds__(kPlaceThreads) void k_region_place(const Entry *in, u64 capr, const u32 *rcount,
                                                                 u32 nreg, u32 shift, u32 nbin, const u32 *bm,
-                                                                u32 bstride, const u64 *boff, Entry *out) {
+                                                                u32 bstride, const u64 *total, u64 *off, Entry *out) {
     // the chunk's entries by field (8-byte words: an entry's place is random,
     // and a 32-byte store per lane to random places conflicts on the LDS
     // banks far more than four 8-byte ones)
     __shared__ u64 sh[kPlaceChunk], sc[kPlaceChunk];
     __shared__ double sre[kPlaceChunk], sim[kPlaceChunk];
-    __shared__ u32 cnt[kRangeBins], lst[kRangeBins];
+    __shared__ u32 cnt[kRangeBins];
+    __shared__ u16 lst[kRangeBins];  // (16 bits: two blocks then fit a CU)
     __shared__ u64 cur[kRangeBins];
     __shared__ u64 tmp[kPlaceThreads / kWave + 1];
     constexpr u32 kBinsPer = kRangeBins / kPlaceThreads;
+    static_assert(kBinsPer == 1, "a thread per bucket");
+    u64 all;
+    const u64 boff = block_excl_scan(threadIdx.x < nbin ? total[threadIdx.x] : 0, tmp, all);  // this thread's bucket's
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < nbin) off[threadIdx.x] = boff;
+        if (threadIdx.x == 0) off[nbin] = all;
+    }
     auto digit = [&](u64 key) { return nbin > 1 ? u32(key >> shift) & (nbin - 1) : 0u; };
     for (u32 r = blockIdx.x; r < nreg; r += gridDim.x) {
         __syncthreads();
-        for (u32 i = threadIdx.x; i < nbin; i += kPlaceThreads) cur[i] = boff[i] + bm[u64(r) * bstride + i];
+        if (threadIdx.x < nbin) cur[threadIdx.x] = boff + bm[u64(r) * bstride + threadIdx.x];
         const u32 n = rcount[r];
         const Entry *src = in + u64(r) * capr;
         for (u32 c0 = 0; c0 < n; c0 += kPlaceChunk) {
@@ -1285,7 +1281,7 @@ __global__ __launch_bounds__(kPlaceThreads) void k_region_place(const Entry *in,
 #pragma unroll
             for (u32 q = 0; q < kBinsPer; ++q) {
                 const u32 b = threadIdx.x * kBinsPer + q;
-                if (b < nbin) lst[b] = u32(run);
+                if (b < nbin) lst[b] = u16(run);
                 run += v[q];
             }
             __syncthreads();

@@ -23,6 +23,7 @@
 #include "qd_k_fastgen.hpp"
 #include "qd_k_finalize.hpp"
 #include "qd_k_generate.hpp"
+#include "qd_k_scan.hpp"
 #include "qd_k_select.hpp"
 
 namespace qd {
@@ -34,52 +35,6 @@ __global__ __launch_bounds__(256) void k_lean_clear(u64 *a, u64 na, u64 *b, u64 
         if (i < na) a[i] = 0;
         else b[i - na] = 0;
     }
-}
-
-// ---------------------------------------------------------------------------
-// decoupled look-back: the exclusive prefix of a tile's aggregate over the
-// tiles before it.  desc[t] = status << 62 | value, cleared before the launch;
-// tiles are handed out by an atomic ticket, so every tile before this one has
-// started, and each publishes its aggregate before it waits for anything:
-// the wait below always ends.  Status and value are one word, so no fence
-// orders them.  Called by the 64 lanes of one wavefront.
-// ---------------------------------------------------------------------------
-constexpr u64 kDescAgg = 1ull << 62, kDescPre = 2ull << 62, kDescVal = (1ull << 62) - 1;
-
-__device__ inline u64 lookback(u64 *desc, u32 tile, u64 agg) {
-    const u32 lane = threadIdx.x & (kWave - 1);
-    if (tile == 0) {
-        if (lane == 0) __hip_atomic_store(desc, kDescPre | agg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return 0;
-    }
-    if (lane == 0) __hip_atomic_store(desc + tile, kDescAgg | agg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    u64 excl = 0;
-    for (i64 top = i64(tile) - 1;; top -= kWave) {
-        const i64 t = top - i64(lane);
-        u64 v = kDescPre;  // before the first tile: the empty prefix
-        u64 have;
-        do {
-            if (t >= 0) v = __hip_atomic_load(desc + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            have = __ballot((v >> 62) != 0);
-        } while (~have);
-        const u64 pre = __ballot((v >> 62) == 2);
-        const u32 stop = pre ? u32(__ffsll((unsigned long long)pre) - 1) : u32(kWave - 1);
-        u64 s = lane <= stop ? (v & kDescVal) : 0;
-#pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1) s += __shfl_xor(s, d, kWave);
-        excl += s;
-        if (pre) break;
-    }
-    if (lane == 0)
-        __hip_atomic_store(desc + tile, kDescPre | (excl + agg), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return excl;
-}
-
-// The next tile of a look-back kernel, for the whole block.
-__device__ inline u32 next_tile(u32 *ticket, u32 *slot) {
-    if (threadIdx.x == 0) *slot = atomicAdd(ticket, 1u);
-    __syncthreads();
-    return *slot;
 }
 
 // ---------------------------------------------------------------------------
@@ -126,7 +81,7 @@ __global__ __launch_bounds__(kScanThreads) void k_lean_scan(const u32 *nc, const
     __shared__ u64 tmp[kScanThreads / kWave + 1], tmp2[kScanThreads / kWave + 1];
     __shared__ u64 pre[2];
     __shared__ u32 slot;
-    const u32 tile = next_tile(&lp->ticket[0], &slot);
+    const u32 tile = next_tile(&lp->ticket[0], 0, &slot);
     const u64 base = u64(tile) * kScanTile + u64(threadIdx.x) * kScanItems;
     u32 v[kScanItems], w[kScanItems];
     u64 s = 0, sw = 0;
@@ -142,10 +97,10 @@ __global__ __launch_bounds__(kScanThreads) void k_lean_scan(const u32 *nc, const
     u64 runw = block_excl_scan(sw, tmp2, totalw);
     // one wavefront looks back for each prefix
     if (threadIdx.x < kWave) {
-        const u64 e = lookback(dc, tile, total);
+        const u64 e = lookback<kWideVal>(dc, tile, total, 0);
         if (threadIdx.x == 0) pre[0] = e;
     } else if (threadIdx.x < 2 * kWave) {
-        const u64 e = lookback(dw, tile, totalw);
+        const u64 e = lookback<kWideVal>(dw, tile, totalw, 0);
         if (threadIdx.x == kWave) pre[1] = e;
     }
     __syncthreads();
@@ -540,7 +495,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_lean_emit(Parents P, const u64
     const u32 ntile = u32((C + kEmitTile - 1) / kEmitTile);
     const u32 lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     for (;;) {
-        const u32 tile = next_tile(&lp->ticket[1], &slot);
+        const u32 tile = next_tile(&lp->ticket[1], 0, &slot);
         if (tile >= ntile) return;
         const u64 c0 = u64(tile) * kEmitTile;
         u32 v[kPer];
@@ -598,10 +553,10 @@ __global__ __launch_bounds__(kEmitThreads) void k_lean_emit(Parents P, const u64
             run += lsize[q] + align_pad(lsize[q], align);
         }
         if (wid == 0) {
-            const u64 e = lookback(dk, tile, cnt);
+            const u64 e = lookback<kWideVal>(dk, tile, cnt, 0);
             if (lane == 0) pre[0] = e;
         } else if (wid == 1) {
-            const u64 e = lookback(db, tile, total);
+            const u64 e = lookback<kWideVal>(db, tile, total, 0);
             if (lane == 0) pre[1] = e;
         }
         __syncthreads();

@@ -58,9 +58,14 @@ __global__ __launch_bounds__(256) void k_scatter1(const u64 *H0, const double2 *
 // Second pass, one workgroup per first-level bucket, splitting it by the
 // next b2 hash bits in one read: sub-bucket d of bucket b owns cap2 slots at
 // ((b << b2) + d) * cap2; workgroup-local cursors place the entries, and the
-// final counts go to cnt2.  A sub-bucket that would exceed cap2 raises
-// ERR_SPILL (the step then repeats this pass with exact counts).
+// final counts go to cnt2.  Entries beyond a sub-bucket's capacity go to the
+// overflow list ovf (*ovf_n of them), where k_dedup_big finds them: a hash
+// that hundreds of candidates share overflows a sub-bucket or two of
+// hundreds of thousands, and repeating the pass for them cost a 12-node
+// split_merge step of 3.2e8 candidates 10.7 ms.  A full list (or none)
+// raises ERR_SPILL, and the step repeats this pass with exact counts.
 constexpr u32 ERR_SPILL = 16u;
+constexpr u64 kOvfCap = 1ull << 16;
 
 // Input bucket b holds off1[b+1] - off1[b] entries, read from in at
 // b * in_stride (fixed-capacity first pass) or at off1[b] (in_stride 0).
@@ -68,7 +73,7 @@ constexpr u32 ERR_SPILL = 16u;
 // group of them: the caller offsets in and off1 to the group's first).
 __global__ __launch_bounds__(1024) void k_level2_fixed(const Entry *in, u64 in_stride, const u64 *off1, u64 nbk1,
                                                        u32 b1, u32 b2, u64 cap2, Entry *out, u64 *cnt2, u32 *err,
-                                                       LeanPlan *lp) {
+                                                       Entry *ovf, u64 *ovf_n, LeanPlan *lp) {
     if (lp) {  // a step driven from the device: off1 holds the buckets' counts
         if (lean_stopped(lp, LEAN_LEVEL2) || lp->b2 == 0) return;
         in_stride = lp->cap1;
@@ -141,6 +146,7 @@ __global__ __launch_bounds__(1024) void k_level2_fixed(const Entry *in, u64 in_s
                 }
             }
             __syncthreads();
+            u32 over = 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const u64 i = cbase + threadIdx.x + 1024 * k;
@@ -157,15 +163,24 @@ __global__ __launch_bounds__(1024) void k_level2_fixed(const Entry *in, u64 in_s
                         dst[2 * at] = lo;
                         dst[2 * at + 1] = hi;
                     } else {
-                        spill = true;
+                        over |= 1u << k;
                     }
                 }
+            }
+            // (apart from the stores above: an atomic among them made every
+            // chunk wait for it, 24 % of the pass; read again from in)
+            while (over) {
+                const u32 k = u32(__builtin_ctz(over));
+                over &= over - 1;
+                const u64 at = ovf ? atomicAdd(reinterpret_cast<unsigned long long *>(ovf_n), 1ull) : kOvfCap;
+                if (at < kOvfCap) ovf[at] = in[ibase + (cbase - beg) + threadIdx.x + 1024 * k];
+                else spill = true;
             }
             __syncthreads();
             for (u32 i = threadIdx.x; i < nb2; i += blockDim.x) cur[i] += ccnt[i];
         }
         __syncthreads();
-        for (u32 i = threadIdx.x; i < nb2; i += blockDim.x) cnt2[(b << b2) + i] = min<u64>(cur[i], cap2);
+        for (u32 i = threadIdx.x; i < nb2; i += blockDim.x) cnt2[(b << b2) + i] = ovf ? cur[i] : min<u64>(cur[i], cap2);
         __syncthreads();  // cur is cleared for the next bucket
     }
     if (spill) atomicOr(err, lp ? LEAN_SPILL : ERR_SPILL);

@@ -40,6 +40,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/quids_hip.h"
@@ -225,6 +226,7 @@ struct qd_ctx {
     // defaults: what quids_amd.tuning picked on the 12-node QCGD workload
     qd_tuning tune = {512, 8, 256, 16384, 1024, 0, 0, 0, 0, 0};
     u64 phase_calls[QD_NUM_PHASES] = {};
+    u32 scan_epoch = 0, scan_ticket = 0;  // of the scans' buffer (run_scan)
     u64 *host = nullptr;  // pinned readback area, 8192 u64
     // scratch of the step
     DBuf nc, cb, pre, tab, kept, keys;
@@ -248,6 +250,7 @@ struct qd_ctx {
                                                 // children's slice tags, per-block bucket counts, group offsets,
     DBuf rcnt, abuf;                            // region counts, a group's merged first-level buckets
     DBuf slab;  // one allocation kept across hash-range steps, carved into their big buffers (views)
+    DBuf ovf;  // the second pass's overflow list
     DBuf lean, ctab, delta;  // the device-driven step: plan, chunks' first parents, child size differences
     DBuf usize, uscr;  // user rules: every candidate's child size, the generate's child bytes
     // output buffers of batched chunks (objects, begin, size, mag per chunk),
@@ -265,7 +268,7 @@ struct qd_ctx {
                 &biglist, &redolist, &bigsoff, &bigkey, &bigcand, &bigmag, &bigseg, &pdesc, &wi, &wb, &cpar, &opar, &ebuf2, &cnt2, &slist, &ukey, &selloop, &segloop, &bsoff, &bscnt,
                 &adjk, &adjv, &adjg, &adjd, &adjp, &adjw, &bseg, &boseg, &brules, &bsinst, &bcount, &bsel, &btrunc,
                 &blist, &bcur, &btile, &bhist, &bkseg, &bchunk, &bcsum, &btot, &pool0, &pool1, &pwpre, &blist2, &mw, &rpart[0], &rpart[1], &rpart[2],
-                &rpart[3], &pk0, &pk1, &tags, &bmat, &goff, &rcnt, &abuf, &slab, &usize, &uscr, &lean, &ctab, &delta};
+                &rpart[3], &pk0, &pk1, &tags, &bmat, &goff, &rcnt, &abuf, &slab, &usize, &uscr, &lean, &ctab, &delta, &ovf};
     }
     void set_names() {
         static const char *const names[] = {
@@ -276,10 +279,10 @@ struct qd_ctx {
             "bseg", "boseg", "brules", "bsinst", "bcount", "bsel", "btrunc", "blist", "bcur", "btile", "bhist",
             "bkseg", "bchunk", "bcsum", "btot", "pool0", "pool1", "pwpre", "blist2", "mw", "rpart0", "rpart1",
             "rpart2", "rpart3", "pk0", "pk1", "tags", "bmat", "goff", "rcnt", "abuf", "slab", "usize", "uscr", "lean",
-            "ctab", "delta"};
+            "ctab", "delta", "ovf"};
         std::vector<DBuf *> v = all_named();
         constexpr size_t kNames = sizeof(names) / sizeof(names[0]);
-        static_assert(kNames == 84, "one name per buffer");
+        static_assert(kNames == 85, "one name per buffer");
         for (size_t i = 0; i < v.size() && i < kNames; ++i) v[i]->name = names[i];
     }
 };
@@ -305,12 +308,27 @@ static int run_scan(qd_ctx *ctx, Load ld, u64 n, u64 *out) {
         return QD_OK;
     }
     const u64 nb = (n + kScanTile - 1) / kScanTile;
-    QD_TRY(ctx->scanblk.ensure(nb * sizeof(u64)));
+    // scanblk: the ticket, then a word per tile; all zero when made and when
+    // the epochs wrap (child counts: for every scan)
+    constexpr bool kWide = std::is_same<Load, LoadU32>::value;
+    const bool made = (nb + 1) * sizeof(u64) > ctx->scanblk.cap || !ctx->scanblk.p;
+    QD_TRY(ctx->scanblk.ensure((nb + 1) * sizeof(u64)));
+    if (kWide || made || ctx->scan_epoch + 1 >= (1u << kEpochBits)) {
+        QD_HIP(hipMemsetAsync(ctx->scanblk.p, 0, kWide && !made ? (nb + 1) * sizeof(u64) : ctx->scanblk.cap,
+                              ctx->stream));
+        ctx->scan_epoch = kWide ? 1u << kEpochBits : 0u;  // (wide words are not epochs': the next scan clears)
+        ctx->scan_ticket = 0;
+    }
     u64 *bs = ctx->scanblk.as<u64>();
-    hipLaunchKernelGGL(k_scan_reduce<Load>, dim3(nb), dim3(kScanThreads), 0, ctx->stream, ld, n, bs);
-    hipLaunchKernelGGL(k_scan_bsums, dim3(1), dim3(1024), 0, ctx->stream, bs, nb);
-    hipLaunchKernelGGL(k_scan_final<Load>, dim3(nb), dim3(kScanThreads), 0, ctx->stream, ld, n, bs, out);
-    QD_HIP(hipGetLastError());
+    hipLaunchKernelGGL((k_scan<Load, kWide ? kWideVal : kShortVal>), dim3(unsigned(nb)), dim3(kScanThreads), 0,
+                       ctx->stream, ld, n, out, reinterpret_cast<u32 *>(bs), ctx->scan_ticket, bs + 1,
+                       kWide ? 0u : ++ctx->scan_epoch);
+    ctx->scan_ticket += u32(nb);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        ctx->scanblk.release();  // (the ticket may not be where the next scan would expect it)
+        return fail(QD_ERR_HIP, std::string("scan: ") + hipGetErrorString(e));
+    }
     return QD_OK;
 }
 
@@ -629,30 +647,33 @@ static int select_topk(qd_ctx *ctx, const u64 *UH, const u64 *UR, const double2 
     return select_loop(ctx, S0, S1, ns, r, 24, bitmap, UR, sbm);
 }
 
-// Buckets beyond the LDS capacity: one workgroup each on global scratch.
-static int dedup_big_buckets(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *boff, u64 nbig, double tol, u64 *UH, u64 *UR,
-                             double2 *UM, u32 *UK, u64 *U) {
+// Buckets beyond the dedup's capacity: one workgroup each on global scratch;
+// novf of their entries in the overflow list.
+static int dedup_big_buckets(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *boff, u64 nbk, u32 L, u64 nbig,
+                             u64 novf, double tol, u64 *UH, u64 *UR, double2 *UM, u32 *UK, u64 *U) {
     hipStream_t s = ctx->stream;
-    std::vector<u64> list(nbig), soff(nbig + 1, 0);
-    QD_TRY(sync_read(ctx, ctx->biglist.p, nbig * sizeof(u64), list.data()));
+    std::vector<u64> cnt(nbig), soff(nbig + 1, 0);
+    QD_TRY(ctx->bigsoff.ensure((nbig + 1) * sizeof(u64)));
+    hipLaunchKernelGGL(k_big_counts, dim3(grid_for(nbig)), dim3(256), 0, s, boff, (const u64 *)ctx->biglist.as<u64>(),
+                       nbig, ctx->bigsoff.as<u64>());
+    QD_HIP(hipGetLastError());
+    QD_TRY(sync_read(ctx, ctx->bigsoff.p, nbig * sizeof(u64), cnt.data()));
     for (u64 q = 0; q < nbig; ++q) {
-        u64 be[2];
-        QD_TRY(sync_read(ctx, boff + list[q], 2 * sizeof(u64), be));
         u64 npad = 2;
-        while (npad < be[1] - be[0]) npad <<= 1;
+        while (npad < cnt[q]) npad <<= 1;
         soff[q + 1] = soff[q] + npad;
     }
     const u64 tot = soff[nbig];
-    QD_TRY(ctx->bigsoff.ensure((nbig + 1) * sizeof(u64)));
     QD_TRY(ctx->bigkey.ensure(tot * sizeof(u64)));
     QD_TRY(ctx->bigcand.ensure(tot * sizeof(u64)));
     QD_TRY(ctx->bigmag.ensure(tot * sizeof(double2)));
     QD_TRY(ctx->bigseg.ensure(tot * sizeof(u32)));
     QD_HIP(hipMemcpyAsync(ctx->bigsoff.p, soff.data(), (nbig + 1) * sizeof(u64), hipMemcpyHostToDevice, s));
     u64 *counters = ctx->counters.as<u64>();
-    hipLaunchKernelGGL(k_dedup_big, dim3(nbig), dim3(1024), 0, s, D, rstride, boff, ctx->biglist.as<u64>(),
-                       ctx->bigsoff.as<u64>(), ctx->bigkey.as<u64>(), ctx->bigcand.as<u64>(), ctx->bigmag.as<double2>(),
-                       ctx->bigseg.as<u32>(), tol, UH, UR, UM, UK, counters, ctx->nhist.as<u64>());
+    hipLaunchKernelGGL(k_dedup_big, dim3(nbig), dim3(1024), 0, s, D, rstride, (const Entry *)ctx->ovf.as<Entry>(), novf,
+                       L, nbk, boff, (const u64 *)ctx->biglist.as<u64>(), (const u64 *)ctx->bigsoff.as<u64>(),
+                       ctx->bigkey.as<u64>(), ctx->bigcand.as<u64>(), ctx->bigmag.as<double2>(), ctx->bigseg.as<u32>(),
+                       tol, UH, UR, UM, UK, counters, ctx->nhist.as<u64>());
     QD_HIP(hipGetLastError());
     QD_TRY(sync_read(ctx, counters, sizeof(u64), U));
     return QD_OK;
@@ -750,13 +771,15 @@ static int ensure_relieved(qd_ctx *ctx, DBuf &b, size_t bytes) {
 // entries, with key bits L above the buckets' LDS home slots and tables of
 // dcap entries: the uniques go to the n slots UH / UR / UM (and UK), U
 // counts them.  Counters 0 and 4..6 of the context must be zero.
+// With spilled, a full overflow list of the pass before (ERR_SPILL) is
+// reported there, and the buckets handed back are left alone.
 static int dedup_phase(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *woff, u64 nbk, u32 L, double tol, u32 dcap,
-                       u64 n, u64 *UH, u64 *UR, double2 *UM, u32 *UK, u64 &U) {
+                       u64 n, u64 *UH, u64 *UR, double2 *UM, u32 *UK, u64 &U, bool *spilled = nullptr) {
     hipStream_t s = ctx->stream;
     u64 *counters = ctx->counters.as<u64>();
     u64 *hb = ctx->host;
     prof_begin(ctx, QD_PHASE_DEDUP);
-    QD_TRY(ctx->biglist.ensure((n / dcap + 2) * sizeof(u64)));
+    QD_TRY(ctx->biglist.ensure((n / (rstride ? std::min<u64>(rstride, dcap) : dcap) + 2) * sizeof(u64)));
     QD_TRY(ctx->redolist.ensure((nbk + 1) * sizeof(u64)));
     int ncu = 256;
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device);
@@ -789,9 +812,13 @@ static int dedup_phase(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *woff
     else if (dcap == 1024) QD_TRY(run_dedup(k_dedup<512, 1024, 2048>, 512));
     else QD_TRY(run_dedup(k_dedup<1024, 2048, 4096>, 1024));
     prof_end(ctx, QD_PHASE_DEDUP);
-    QD_HIP(hipMemcpyAsync(hb, counters, 7 * sizeof(u64), hipMemcpyDeviceToHost, s));
+    QD_HIP(hipMemcpyAsync(hb, counters, 9 * sizeof(u64), hipMemcpyDeviceToHost, s));
     QD_HIP(hipStreamSynchronize(s));
     prof_collect(ctx);
+    if (spilled) {
+        *spilled = u32(hb[4]) & ERR_SPILL;
+        if (*spilled) return QD_OK;
+    }
     if (hb[6]) {
         prof_begin(ctx, QD_PHASE_DEDUP);
         if (dcap == 256) QD_TRY(run_sort(k_dedup_sort<128, 256, 512>, 128, hb[6]));
@@ -799,13 +826,14 @@ static int dedup_phase(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *woff
         else if (dcap == 1024) QD_TRY(run_sort(k_dedup_sort<512, 1024, 2048>, 512, hb[6]));
         else QD_TRY(run_sort(k_dedup_sort<1024, 2048, 4096>, 1024, hb[6]));
         prof_end(ctx, QD_PHASE_DEDUP);
-        QD_HIP(hipMemcpyAsync(hb, counters, 7 * sizeof(u64), hipMemcpyDeviceToHost, s));
+        QD_HIP(hipMemcpyAsync(hb, counters, 9 * sizeof(u64), hipMemcpyDeviceToHost, s));
         QD_HIP(hipStreamSynchronize(s));
         prof_collect(ctx);
     }
     QD_TRY(check_err_word(u32(hb[4])));
     U = hb[0];
-    if (hb[5]) QD_TRY(dedup_big_buckets(ctx, D, rstride, woff, hb[5], tol, UH, UR, UM, UK, &U));
+    if (hb[5])
+        QD_TRY(dedup_big_buckets(ctx, D, rstride, woff, nbk, L, hb[5], rstride ? hb[7] : 0, tol, UH, UR, UM, UK, &U));
     return QD_OK;
 }
 
@@ -872,6 +900,7 @@ static int partition_dedup(qd_ctx *ctx, const u64 *H0, const double2 *M0, const 
         if (wide2 > cap2 && nb * wide2 <= std::max<u64>(full2, n)) cap2 = wide2;
         QD_TRY(ctx->off2.ensure((nb + 1) * sizeof(u64)));
         QD_TRY(ctx->cnt2.ensure(nb * sizeof(u64)));
+        QD_TRY(ctx->ovf.ensure(kOvfCap * sizeof(Entry)));
         // fixed-capacity sub-buckets unless their padding would pass the
         // pass budget's buffer (small sub-buckets near the budget): then
         // exact offsets from a counting pass
@@ -888,7 +917,7 @@ static int partition_dedup(qd_ctx *ctx, const u64 *H0, const double2 *M0, const 
             (void)hipDeviceGetAttribute(&ncu2, hipDeviceAttributeMultiprocessorCount, ctx->device);
             const unsigned g2 = unsigned(std::min<u64>(nb1, std::max(ncu2 / 2, 1)));
             hipLaunchKernelGGL(k_level2_fixed, dim3(g2), dim3(1024), 0, s, (const Entry *)E1, in_stride,
-                               ctx->off1.as<u64>(), nb1, b1, b2, cap2, E2, ctx->cnt2.as<u64>(), errw, (LeanPlan *)nullptr);
+                               ctx->off1.as<u64>(), nb1, b1, b2, cap2, E2, ctx->cnt2.as<u64>(), errw, ctx->ovf.as<Entry>(), counters + 7, (LeanPlan *)nullptr);
             QD_HIP(hipGetLastError());
             QD_TRY(run_scan(ctx, LoadU64{ctx->cnt2.as<u64>()}, nb, ctx->off2.as<u64>()));
             QD_TRY(sync_read(ctx, errw, sizeof(u32), &ew));
@@ -1479,6 +1508,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
     QD_TRY(ctx->bmat.ensure(u64(gr) * nb1 * sizeof(u32)));
     QD_TRY(ctx->off1.ensure((nb1 + 1) * sizeof(u64)));
     QD_TRY(ctx->cnt2.ensure(nb2g * sizeof(u64)));
+    QD_TRY(ctx->ovf.ensure(kOvfCap * sizeof(Entry)));
     QD_TRY(ctx->off2.ensure((nb2g + 1) * sizeof(u64)));
     QD_TRY(carve(ctx->pool0, pcap * 32));
     QD_TRY(carve(ctx->pool1, (capped ? max_obj + 1 : 1) * 32));
@@ -1527,6 +1557,8 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
         QD_HIP(hipMemcpyAsync(Pr, Qr, max_obj * sizeof(u64), hipMemcpyDeviceToDevice, s));
         QD_HIP(hipMemcpyAsync(Pm, Qm, max_obj * sizeof(double2), hipMemcpyDeviceToDevice, s));
         if (ukeys) QD_HIP(hipMemcpyAsync(Pk, Qk, max_obj * sizeof(u32), hipMemcpyDeviceToDevice, s));
+        hb[kHostN - 1] = max_obj;
+        QD_HIP(hipMemcpyAsync(pcount, hb + kHostN - 1, sizeof(u64), hipMemcpyHostToDevice, s));
         prof_end(ctx, QD_PHASE_SELECT);
         ns = max_obj;
         if (ukeys && !sk.prob) t24 = std::max(t24, c24);
@@ -1568,13 +1600,18 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
                                (const u64 *)ctx->tab.as<u64>(), P.begin, rule, nitems, rs, gbits, GB, capr,
                                ctx->rcnt.as<u32>(), b1, ctx->bmat.as<u32>(), errw);
             QD_HIP(hipGetLastError());
+            // every block's first place in each first-level bucket, and the
+            // buckets' sizes
+            hipLaunchKernelGGL(k_range_colscan, dim3(unsigned(nb1)), dim3(256), 0, s, ctx->bmat.as<u32>(), u32(gr),
+                               u32(nb1), u32(nb1), ctx->cur1.as<u64>());
+            QD_HIP(hipGetLastError());
             prof_end(ctx, QD_PHASE_GENERATE);
             u32 ew = 0;
+            QD_HIP(hipMemcpyAsync(rc.data(), ctx->rcnt.p, rc.size() * sizeof(u32), hipMemcpyDeviceToHost, s));
             QD_TRY(sync_read(ctx, errw, sizeof(u32), &ew));
             single = !(ew & ERR_SPILL1);
         }
         if (single) {
-            QD_TRY(sync_read(ctx, ctx->rcnt.p, rc.size() * sizeof(u32), rc.data()));
             u64 kept = 0;
             for (u32 v : rc) kept += v;
             if (kept != n) return fail(QD_ERR_HIP, "hash-range pass kept a different candidate count than it counted");
@@ -1645,17 +1682,10 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
                     return fail(QD_ERR_CAPACITY, "hash-range pass: hash keys too skewed for the first radix pass");
                 const u32 *rcg = ctx->rcnt.as<u32>() + u64(g) * gr;
                 prof_begin(ctx, QD_PHASE_PARTITION);
-                // the walk counted each block's children per first-level
-                // bucket (row = block, nb1 columns): the group's columns
-                u32 *bmg = ctx->bmat.as<u32>() + u64(g) * gbk;
-                hipLaunchKernelGGL(k_range_colscan, dim3(unsigned(gbk)), dim3(256), 0, s, bmg, u32(gr), u32(gbk),
-                                   u32(nb1), ctx->cur1.as<u64>());
-                hipLaunchKernelGGL(k_excl_small, dim3(1), dim3(64), 0, s, (const u64 *)ctx->cur1.as<u64>(), u32(gbk),
-                                   ctx->off1.as<u64>());
-                hipLaunchKernelGGL(k_region_place, dim3(gr), dim3(kPlaceThreads), 0, s, (const Entry *)GB.g[g], capr, rcg,
-                                   u32(gr),
-                                   64 - b1, u32(gbk), (const u32 *)bmg, u32(nb1), (const u64 *)ctx->off1.as<u64>(),
-                                   ctx->abuf.as<Entry>());
+                const u64 g0 = u64(g) * gbk;  // the group's first bucket: its columns of bmat
+                hipLaunchKernelGGL(k_region_place, dim3(gr), dim3(kPlaceThreads), 0, s, (const Entry *)GB.g[g], capr,
+                                   rcg, u32(gr), 64 - b1, u32(gbk), (const u32 *)ctx->bmat.as<u32>() + g0, u32(nb1),
+                                   (const u64 *)ctx->cur1.as<u64>() + g0, ctx->off1.as<u64>(), ctx->abuf.as<Entry>());
                 QD_HIP(hipGetLastError());
                 prof_end(ctx, QD_PHASE_PARTITION);
                 gin = ctx->abuf.as<Entry>();
@@ -1675,30 +1705,34 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
             Entry *E2 = ctx->ebuf2.as<Entry>();
             QD_HIP(hipMemsetAsync(counters, 0, 8 * sizeof(u64), s));
             u64 rstride = 0;
-            prof_begin(ctx, QD_PHASE_PARTITION);
-            if (b2) {
-                bool exact = l2_exact;
-                if (!exact) {
+            u64 *UH = reinterpret_cast<u64 *>(ub), *UR = UH + ng;
+            double2 *UM = reinterpret_cast<double2 *>(UR + ng);
+            u32 *UK = ukeys ? ctx->ukey.as<u32>() : nullptr;
+            u64 U = 0;
+            for (;;) {
+                const bool exact = l2_exact;
+                prof_begin(ctx, QD_PHASE_PARTITION);
+                if (b2 && !exact) {
                     int ncu2 = 256;
                     (void)hipDeviceGetAttribute(&ncu2, hipDeviceAttributeMultiprocessorCount, ctx->device);
                     const unsigned g2 = unsigned(std::min<u64>(gbk, std::max(ncu2 / 2, 1)));
                     hipLaunchKernelGGL(k_level2_fixed, dim3(g2), dim3(1024), 0, s, gin, u64(0), go, gbk, b1, b2, cap2,
-                                       E2, ctx->cnt2.as<u64>(), errw, (LeanPlan *)nullptr);
+                                       E2, ctx->cnt2.as<u64>(), errw, ctx->ovf.as<Entry>(), counters + 7,
+                                       (LeanPlan *)nullptr);
                     QD_HIP(hipGetLastError());
                     QD_TRY(run_scan(ctx, LoadU64{ctx->cnt2.as<u64>()}, nb2g, ctx->off2.as<u64>()));
-                    u32 ew2 = 0;
-                    QD_TRY(sync_read(ctx, errw, sizeof(u32), &ew2));
                     rstride = cap2;
-                    if (ew2 & ERR_SPILL) {
-                        QD_HIP(hipMemsetAsync(errw, 0, sizeof(u32), s));
-                        exact = true;
-                        // a rule whose hashes repeat enough to spill once
-                        // (split_merge) spills in most groups: exact offsets
-                        // from here on
-                        l2_exact = true;
+                    if (!single) {  // (the uniques will overwrite gin: look before the dedup)
+                        u32 ew2 = 0;
+                        QD_TRY(sync_read(ctx, errw, sizeof(u32), &ew2));
+                        if (ew2 & ERR_SPILL) {
+                            l2_exact = true;
+                            QD_HIP(hipMemsetAsync(counters, 0, 8 * sizeof(u64), s));
+                            prof_end(ctx, QD_PHASE_PARTITION);
+                            continue;
+                        }
                     }
-                }
-                if (exact) {  // a sub-bucket passed its capacity: exact offsets
+                } else if (b2) {
                     hb[kHostN] = ng;
                     QD_HIP(hipMemcpyAsync(ctx->off2.as<u64>() + nb2g, hb + kHostN, sizeof(u64),
                                           hipMemcpyHostToDevice, s));
@@ -1707,35 +1741,38 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
                     QD_HIP(hipGetLastError());
                     rstride = 0;
                     st.reserved |= 1;
+                } else {
+                    // one level: the group's first-pass buckets are the dedup's
+                    QD_HIP(hipMemcpyAsync(E2, gin + obase, ng * sizeof(Entry), hipMemcpyDeviceToDevice, s));
+                    hipLaunchKernelGGL(k_add_offset, dim3(grid_for(gbk + 1)), dim3(256), 0, s, go, gbk + 1,
+                                       u64(0) - obase, ctx->off2.as<u64>());
+                    QD_HIP(hipGetLastError());
                 }
-            } else {
-                // one level: the group's first-pass buckets are the dedup's
-                QD_HIP(hipMemcpyAsync(E2, gin + obase, ng * sizeof(Entry), hipMemcpyDeviceToDevice, s));
-                hipLaunchKernelGGL(k_add_offset, dim3(grid_for(gbk + 1)), dim3(256), 0, s, go, gbk + 1, u64(0) - obase,
-                                   ctx->off2.as<u64>());
-                QD_HIP(hipGetLastError());
+                prof_end(ctx, QD_PHASE_PARTITION);
+                bool spilled = false;
+                QD_TRY(dedup_phase(ctx, E2, rstride, ctx->off2.as<u64>(), b2 ? nb2g : gbk, b1 + b2, prm.tolerance, dcap,
+                                   ng, UH, UR, UM, UK, U, &spilled));
+                if (!spilled) break;
+                // the overflow list did not hold what the sub-buckets could
+                // not: a rule whose hashes repeat that much does so in most
+                // groups, so exact offsets from here on (gin, the group's
+                // merged buckets, is still whole; the uniques overwrite its
+                // regions)
+                l2_exact = true;
+                QD_HIP(hipMemsetAsync(counters, 0, 8 * sizeof(u64), s));
             }
-            prof_end(ctx, QD_PHASE_PARTITION);
-            u64 *UH = reinterpret_cast<u64 *>(ub), *UR = UH + ng;
-            double2 *UM = reinterpret_cast<double2 *>(UR + ng);
-            u32 *UK = ukeys ? ctx->ukey.as<u32>() : nullptr;
-            u64 U = 0;
-            QD_TRY(dedup_phase(ctx, E2, rstride, ctx->off2.as<u64>(), b2 ? nb2g : gbk, b1 + b2, prm.tolerance, dcap,
-                               ng, UH, UR, UM, UK, U));
             Utot += U;
+            ns = hb[8];  // the pool as the groups before this one left it
             if (!U) continue;
-            if (capped && ns + ng > pcap) QD_TRY(trim_pool());
-            hb[kHostN - 1] = ns;
-            QD_HIP(hipMemcpyAsync(pcount, hb + kHostN - 1, sizeof(u64), hipMemcpyHostToDevice, s));
+            if (capped && (ns > 2 * max_obj || ns + ng > pcap)) QD_TRY(trim_pool());
             hipLaunchKernelGGL(k_pool_append,
                                dim3(unsigned(std::min<u64>((ng + 256 * kPoolPer - 1) / (256 * kPoolPer), 16384))),
                                dim3(256), 0, s, (const u64 *)UH, (const u64 *)UR, (const double2 *)UM, (const u32 *)UK,
                                t24, ng, Ph, Pr, Pm, Pk, pcount);
             QD_HIP(hipGetLastError());
-            QD_TRY(sync_read(ctx, pcount, sizeof(u64), &ns));
-            if (capped && ns > 2 * max_obj) QD_TRY(trim_pool());
         }
     }
+    QD_TRY(sync_read(ctx, pcount, sizeof(u64), &ns));
     tl[5] = wall_ms();
     phase_mark(ctx, PH_TRUNC);
     if (capped && ns > max_obj) QD_TRY(trim_pool());
@@ -2121,7 +2158,7 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, const qd_rule &rule, const L
     prof_begin(ctx, QD_PHASE_PARTITION);
     if (two)
         hipLaunchKernelGGL(k_level2_fixed, dim3(128), dim3(1024), 0, s, (const Entry *)E1, u64(0), (const u64 *)cnt1,
-                           u64(0), 0u, 0u, u64(0), E2, cnt2, (u32 *)nullptr, lp);
+                           u64(0), 0u, 0u, u64(0), E2, cnt2, (u32 *)nullptr, (Entry *)nullptr, (u64 *)nullptr, lp);
     hipLaunchKernelGGL(k_lean_bscan, dim3(1), dim3(1024), 0, s, (const u64 *)cnt1, (const u64 *)cnt2,
                        (const LeanPlan *)lp, ctx->off2.as<u64>());
     QD_HIP(hipGetLastError());

@@ -146,3 +146,26 @@ def test_populate_register_sizes(size):
         g, _ = _step(hs, qc.hadamard(bit), q.UINT64_MAX)
         o, _ = orc.simulate(hs, qc.hadamard(bit))
         assert_states_identical(g, o, f"size {size} bit {bit}")
+
+
+# hashes that hundreds of candidates share, beyond a sub-bucket's fixed
+# capacity: the entries beyond it go through the overflow list; a list that
+# is full makes the pass repeat with exact counts
+@pytest.mark.parametrize("copies,exact", [(690, False), (1500, False), (9000, True)])
+@pytest.mark.parametrize("eager", [0, 1])
+def test_overflowing_sub_buckets(copies, exact, eager):
+    grown = qcgd_initial(12, 42)
+    for r in (qcgd.split_merge(0.7, 0.2), qcgd.erase_create(1.0, 0.4)) * 2:
+        grown = orc.simulate(grown, r, 2500)[0]
+        grown = orc.apply_modifier(grown, qcgd.step)
+    rng = np.random.default_rng(copies)
+    objs = grown.objects_list() + [qcgd.seeded_graph(7, 5)] * copies
+    mags = np.concatenate([grown.magnitude, 0.02 * (rng.normal(size=copies) + 1j * rng.normal(size=copies))])
+    hs = HostState.from_objects(objs, mags)
+    rule = qcgd.erase_create(0.8, 0.3)
+    o, ost = orc.simulate(hs, rule, 20000)
+    assert ost["num_candidates"] > 170000
+    g, st = _step(hs, rule, 20000, eager_select=eager)
+    assert st["num_unique"] == ost["num_unique"]
+    assert bool(st["reserved"] & 1) == exact or st["reserved"] & 8
+    assert_states_identical(g, o, f"copies {copies}")
