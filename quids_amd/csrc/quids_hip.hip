@@ -38,6 +38,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <string>
 #include <type_traits>
@@ -93,13 +94,110 @@ constexpr size_t kBigAlloc = 48ull << 30;
 static double dbuf_ms();
 static void dbuf_log(const char *what, size_t bytes, double ms, const char *name = nullptr);
 
+// State buffers given up (a state closed, or grown) and not yet returned to
+// the device, for the context's next ones: mapping and unmapping 10 MB to
+// 1 GB costs 25-300 us each time, and a program that makes a state per step
+// (the gradient's forward pass) spent a quarter of its time on it.  Bounded
+// (kPoolBytes); given back when an allocation does not fit, when the context
+// is trimmed or destroyed, and before free memory decides anything.
+struct StatePool {
+    struct Buf {
+        void *p;
+        size_t cap;
+    };
+    std::mutex m;
+    std::vector<Buf> bufs;  // oldest first
+    size_t bytes = 0;
+    // the smallest buffer of at least `want` bytes, and at most twice that
+    // (plus 1 MB), or nothing
+    Buf take(size_t want) {
+        std::lock_guard<std::mutex> g(m);
+        size_t best = bufs.size();
+        for (size_t i = 0; i < bufs.size(); ++i)
+            if (bufs[i].cap >= want && bufs[i].cap <= 2 * want + (1 << 20) &&
+                (best == bufs.size() || bufs[i].cap < bufs[best].cap))
+                best = i;
+        if (best == bufs.size()) return {nullptr, 0};
+        const Buf b = bufs[best];
+        bufs.erase(bufs.begin() + long(best));
+        bytes -= b.cap;
+        return b;
+    }
+    // (the device has finished with p: an unmapping would have waited for it,
+    // whatever stream used it)
+    void give(void *p, size_t cap) {
+        constexpr size_t kSmall = 64 << 10;  // the runtime hands these out in a microsecond itself
+        (void)hipDeviceSynchronize();
+        if (cap < kSmall || cap > kPoolBytes / 2) {
+            (void)hipFree(p);
+            return;
+        }
+        std::lock_guard<std::mutex> g(m);
+        while (!bufs.empty() && (bytes + cap > kPoolBytes || bufs.size() >= 64)) {
+            (void)hipFree(bufs.front().p);
+            bytes -= bufs.front().cap;
+            bufs.erase(bufs.begin());
+        }
+        bufs.push_back({p, cap});
+        bytes += cap;
+    }
+    size_t held() {
+        std::lock_guard<std::mutex> g(m);
+        return bytes;
+    }
+    void trim() {
+        std::lock_guard<std::mutex> g(m);
+        for (Buf &b : bufs) (void)hipFree(b.p);
+        bufs.clear();
+        bytes = 0;
+    }
+    static constexpr size_t kPoolBytes = 4ull << 30;
+};
+
+// Every context's pool, for an allocation that does not fit.
+static std::mutex g_pools_m;
+static std::vector<StatePool *> g_pools;
+static void trim_pools() {
+    std::lock_guard<std::mutex> g(g_pools_m);
+    for (StatePool *p : g_pools) p->trim();
+}
+
+// hipMalloc; the pooled state buffers go when it does not fit.
+static hipError_t device_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        trim_pools();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 struct DBuf {
     void *p = nullptr;
     size_t cap = 0;
     bool tight = false;  // grows to the size asked (+1/8), not by 1.5x: the states' buffers
     bool view = false;   // p points into another buffer (the hash-range slab): never freed here
     const char *name = nullptr;  // for the QD_LOG_RANGE allocation log
+    StatePool *pool = nullptr;   // a state's buffer: where it comes from and goes to
+    size_t nominal = 0;          // with a pool: the bytes it would hold if made for the sizes asked alone
+                                 // (what memory-driven truncation counts)
+    // the bytes taken for `bytes`, at the present size
+    size_t policy(size_t bytes, size_t old) const {
+        // a buffer that grows takes at least 1.5x its old size, so steps of
+        // varying size settle on few reallocations; but no more than
+        // kBigAlloc unless asked for it: on MI355X, allocations of 64 GB and
+        // more take seconds to map and to free, smaller ones about 1 ms
+        size_t want = std::max<size_t>(bytes + bytes / 8, 256);
+        if (old && !tight) want = std::max(want, old + old / 2);
+        return std::min(want, std::max(bytes, kBigAlloc));
+    }
+    // accounts for `bytes` in use (with a pool)
+    void account(size_t bytes) {
+        if (bytes > nominal || !nominal) nominal = policy(bytes, nominal);
+    }
     int ensure(size_t bytes) {
+        if (pool) account(bytes);
         if (bytes <= cap && p) return QD_OK;
         if (view) {  // a view that must grow becomes a buffer of its own
             p = nullptr;
@@ -107,22 +205,18 @@ struct DBuf {
             view = false;
         }
         const size_t old = cap;
-        if (p) {
-            const double t0 = dbuf_ms();
-            (void)hipFree(p);
-            dbuf_log("hipFree", cap, dbuf_ms() - t0, name);
-            p = nullptr;
-            cap = 0;
+        drop();
+        size_t want = policy(bytes, old);
+        if (pool) {
+            const StatePool::Buf b = pool->take(want);
+            if (b.p) {
+                p = b.p;
+                cap = b.cap;
+                return QD_OK;
+            }
         }
-        // a buffer that grows takes at least 1.5x its old size, so steps of
-        // varying size settle on few reallocations; but no more than
-        // kBigAlloc unless asked for it: on MI355X, allocations of 64 GB and
-        // more take seconds to map and to free, smaller ones about 1 ms
-        size_t want = std::max<size_t>(bytes + bytes / 8, 256);
-        if (old && !tight) want = std::max(want, old + old / 2);
-        want = std::min(want, std::max(bytes, kBigAlloc));
         double t0 = dbuf_ms();
-        hipError_t e = hipMalloc(&p, want);
+        hipError_t e = device_malloc(&p, want);
         dbuf_log(e == hipSuccess ? "hipMalloc" : "hipMalloc (failed)", want, dbuf_ms() - t0, name);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -139,25 +233,42 @@ struct DBuf {
                                             std::to_string(freeb) + " of " + std::to_string(totalb) + " bytes)");
             }
             want = std::max<size_t>(bytes, 256);
+            nominal = want;
         }
         cap = want;
         return QD_OK;
     }
-    void release() {
+    // gives up what it owns
+    void drop() {
         if (p && !view) {
             const double t0 = dbuf_ms();
-            (void)hipFree(p);
+            if (pool) pool->give(p, cap);
+            else (void)hipFree(p);
             dbuf_log("hipFree", cap, dbuf_ms() - t0, name);
         }
         p = nullptr;
         cap = 0;
+    }
+    void release() {
+        drop();
         view = false;
+        nominal = 0;
+    }
+    // takes a pooled buffer of at least `bytes` in place of a smaller one, if
+    // there is one
+    void grow_from_pool(size_t bytes) {
+        if (!pool || (p && cap >= bytes)) return;
+        const StatePool::Buf b = pool->take(bytes);
+        if (!b.p) return;
+        drop();
+        p = b.p;
+        cap = b.cap;
     }
     // releases, then allocates exactly `bytes`
     int alloc_exact(size_t bytes) {
         release();
         const double t0 = dbuf_ms();
-        const hipError_t e = hipMalloc(&p, bytes);
+        const hipError_t e = device_malloc(&p, bytes);
         dbuf_log(e == hipSuccess ? "hipMalloc" : "hipMalloc (failed)", bytes, dbuf_ms() - t0, name);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -228,6 +339,10 @@ struct qd_ctx {
     u64 phase_calls[QD_NUM_PHASES] = {};
     u32 scan_epoch = 0, scan_ticket = 0;  // of the scans' buffer (run_scan)
     u64 *host = nullptr;  // pinned readback area, 8192 u64
+    StatePool pool;       // its states' buffers between uses
+    size_t total_mem = 0; // of the device
+    u8 *ring = nullptr;   // pinned staging of small uploads (kRing bytes), used round and round
+    size_t ring_at = 0;
     // scratch of the step
     DBuf nc, cb, pre, tab, kept, keys;
     DBuf ebuf0, ebuf1;
@@ -290,6 +405,10 @@ struct qd_ctx {
 struct qd_state {
     qd_ctx *ctx = nullptr;
     DBuf objects{nullptr, 0, true}, begin{nullptr, 0, true}, size{nullptr, 0, true}, mag{nullptr, 0, true};
+    // takes and returns its buffers through the context's pool
+    void use_pool(StatePool *p) {
+        for (DBuf *b : {&objects, &begin, &size, &mag}) b->pool = p;
+    }
     u64 n = 0;
     u64 bytes = 0;
     double total_proba = 1;
@@ -371,9 +490,16 @@ static void phase_mark(qd_ctx *ctx, int upto) {
     for (; ctx->next_phase <= upto; ++ctx->next_phase) ctx->hook(kPhaseNames[ctx->next_phase], ctx->hook_user);
 }
 
+// (small reads through the pinned area: into pageable memory the runtime
+// stages them itself, about 30 us a call)
+constexpr u64 kHostRead = 1024, kHostReadWords = 6144;
 static int sync_read(qd_ctx *ctx, const void *dev, size_t bytes, void *host) {
-    QD_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    u64 *const pinned = ctx->host;
+    const bool own = host >= (void *)pinned && host < (void *)(pinned + 8192);
+    void *to = own || bytes > kHostReadWords * sizeof(u64) ? host : pinned + kHostRead;
+    QD_HIP(hipMemcpyAsync(to, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
     QD_HIP(hipStreamSynchronize(ctx->stream));
+    if (to != host) std::memcpy(host, to, bytes);
     prof_collect(ctx);
     return QD_OK;
 }
@@ -714,7 +840,7 @@ static u64 step_budget(qd_ctx *ctx) {
         (void)hipGetLastError();
         return 1ull << 28;
     }
-    u64 cached = 0;
+    u64 cached = ctx->pool.held();
     for (DBuf *b : ctx->all())
         if (!b->view) cached += b->cap;
     // the largest buffer (the second partition pass, about 1.7 x 32 bytes per
@@ -1041,7 +1167,13 @@ __global__ __launch_bounds__(256) void k_masked_sum(const u64 *w, const u64 *bit
     if ((threadIdx.x & (kWave - 1)) == 0 && acc) atomicAdd(reinterpret_cast<unsigned long long *>(out), acc);
 }
 
-static u64 state_mem(const qd_state *s) { return s->objects.cap + s->begin.cap + s->size.cap + s->mag.cap; }
+// A state's memory as memory-driven truncation counts it: what its sizes ask
+// for, also where a pooled buffer is larger.
+static u64 state_mem(const qd_state *s) {
+    u64 t = 0;
+    for (const DBuf *b : {&s->objects, &s->begin, &s->size, &s->mag}) t += b->pool ? b->nominal : b->cap;
+    return t;
+}
 
 static u64 ctx_scratch(qd_ctx *ctx) {
     u64 t = 0;
@@ -1053,6 +1185,7 @@ static u64 ctx_scratch(qd_ctx *ctx) {
 // Free device memory as memory-driven truncation sees it (the reference
 // reads the host's, src/utils/memory.hpp:25-36), at most free_mem_mib.
 static int free_mem(qd_ctx *ctx, u64 &freeb) {
+    ctx->pool.trim();
     size_t f = 0, total = 0;
     QD_HIP(hipMemGetInfo(&f, &total));
     freeb = f;
@@ -1240,10 +1373,27 @@ static int mem_survivor_cap(qd_ctx *ctx, const Parents &P, const qd_rule &rule, 
 // hash-range passes (qd_k_range.hpp): steps whose candidates exceed the
 // scratch memory
 // ===========================================================================
-// Copies host bytes into a device buffer (grown as needed).
+// Copies host bytes into a device buffer (grown as needed).  Small ones go
+// through the pinned ring and are not waited for (when the ring comes round,
+// the copies before are): a pageable copy and its wait took 20-90 us, and a
+// batched step makes nine.
+constexpr size_t kRing = 1 << 20;
 static int upload(qd_ctx *ctx, DBuf &b, const void *src, size_t bytes) {
     QD_TRY(b.ensure(std::max<size_t>(bytes, 8)));
-    if (bytes) QD_HIP(hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    if (!bytes) return QD_OK;
+    if (bytes <= kRing / 4) {
+        const size_t need = (bytes + 63) / 64 * 64;
+        if (ctx->ring_at + need > kRing) {
+            QD_HIP(hipStreamSynchronize(ctx->stream));
+            ctx->ring_at = 0;
+        }
+        u8 *at = ctx->ring + ctx->ring_at;
+        ctx->ring_at += need;
+        std::memcpy(at, src, bytes);
+        QD_HIP(hipMemcpyAsync(b.p, at, bytes, hipMemcpyHostToDevice, ctx->stream));
+        return QD_OK;
+    }
+    QD_HIP(hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     QD_HIP(hipStreamSynchronize(ctx->stream));  // the host source may go away
     return QD_OK;
 }
@@ -1327,6 +1477,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
                             kSlabSlack * kRangeBytesPerCand * double(budget) + double(64ull << 20);
         slab_want = std::max<u64>(slab_want, u64(need));
     } else {
+        ctx->pool.trim();
         size_t freeb = 0, totalb = 0;
         QD_HIP(hipMemGetInfo(&freeb, &totalb));
         u64 reuse = 0;  // owned buffers the slab replaces
@@ -1337,7 +1488,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
         // the next state with its finalize scratch (Kp objects at 1.5 x the
         // parents' mean size), beyond what the output state holds already
         const double next = std::max(0.0, 1.5 * double(in_bytes) / double(std::max<u64>(N, 1)) * Kp + 60.0 * Kp -
-                                              double(state_mem(out)));
+                                              double(out->objects.cap + out->begin.cap + out->size.cap + out->mag.cap));
         const double fixed = next + double(2ull << 30);
         const double avail = 0.95 * (double(freeb) + double(ctx->slab.cap) + double(reuse)) - fixed;
         // keep the slab while it is within 80-115 % of what would be made now
@@ -2101,7 +2252,7 @@ static bool lean_allowed(qd_ctx *ctx, const SelKey &sk) {
 // them when the host knows (C != 0), else what the scan found.  One wait, at
 // the end; a second one when the output state had to grow.
 template <int KIND>
-static int lean_tail(qd_ctx *ctx, const Parents &P, const qd_rule &rule, const LeanArea &la, u64 room, u64 C,
+static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule &rule, const LeanArea &la, u64 room, u64 C,
                      u64 nitems, u64 max_obj, const qd_params &prm, qd_state *out, qd_step_stats &st, LeanEnd &le) {
     hipStream_t s = ctx->stream;
     u64 *a = ctx->lean.as<u64>();
@@ -2132,6 +2283,12 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, const qd_rule &rule, const L
     u32 *UK = keys ? ctx->ukey.as<u32>() : nullptr;
     u32 *slotof = ctx->ebuf1.as<u32>();  // (after the dedup has read its entries)
     u64 *nhist = a + la.nhist, *hist2 = a + la.hist2, *cnt1 = a + la.cnt1;
+    if (C) {  // a fresh state: pooled buffers of about the size that a truncated step's survivors need
+        out->begin.grow_from_pool((bound + 1) * sizeof(u64));
+        out->size.grow_from_pool(bound * sizeof(u32));
+        out->mag.grow_from_pool(bound * sizeof(double2));
+        out->objects.grow_from_pool(u64(1.2 * double(bound) * (double(in_bytes) / double(P.n) + 8)));
+    }
     u64 *cnt2 = two ? ctx->cnt2.as<u64>() : cnt1;
     const u64 *cb = ctx->cb.as<u64>(), *ctab = ctx->ctab.as<u64>();
     LeanReport *rep = reinterpret_cast<LeanReport *>(ctx->host + kHostLean);
@@ -2236,6 +2393,10 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, const qd_rule &rule, const L
     st.num_survivors = K;
     st.output_bytes = rep->bytes;
     if (K) {
+        out->begin.account((K + 1) * sizeof(u64));
+        out->size.account(K * sizeof(u32));
+        out->mag.account(K * sizeof(double2));
+        out->objects.account(rep->bytes);
         out->n = K;
         out->bytes = rep->bytes;
         out->total_proba = rep->total;
@@ -2390,7 +2551,7 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
         QD_TRY(scan_parents(nullptr));
     }
     if (room) {
-        QD_TRY(lean_tail<KIND>(ctx, P, rule, la, room, 0, 0, max_obj, prm, out, st, le));
+        QD_TRY(lean_tail<KIND>(ctx, P, in_bytes, rule, la, room, 0, 0, max_obj, prm, out, st, le));
     } else {
         QD_HIP(hipStreamSynchronize(s));
         prof_collect(ctx);
@@ -2434,7 +2595,7 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
             QD_HIP(hipGetLastError());
             defer_tab = false;
         }
-        QD_TRY(lean_tail<KIND>(ctx, P, rule, la, C, C, nitems, max_obj, prm, out, st, le));
+        QD_TRY(lean_tail<KIND>(ctx, P, in_bytes, rule, la, C, C, nitems, max_obj, prm, out, st, le));
     }
     if (le.done) {
         u32 b1, b2;
@@ -2653,9 +2814,10 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
 // needs its room.
 static int relieve_memory(qd_ctx *ctx) {
     if (ctx->slab.p) return QD_OK;  // hash-range steps: their buffers are sized and kept on purpose
+    if (ctx_scratch(ctx) <= ctx->total_mem / 4) return QD_OK;  // (asking for the free memory takes 13 us)
     size_t freeb = 0, totalb = 0;
     QD_HIP(hipMemGetInfo(&freeb, &totalb));
-    if (ctx_scratch(ctx) > totalb / 4 && freeb < totalb / 2) {
+    if (freeb < totalb / 2) {
         QD_HIP(hipStreamSynchronize(ctx->stream));
         const std::vector<DBuf *> keep = range_cache(ctx);
         for (DBuf *b : ctx->all())
@@ -2953,7 +3115,7 @@ static int adjoint_kind(qd_ctx *ctx, qd_state *in, const qd_rule &rule, const qd
         QD_HIP(hipGetLastError());
         QD_TRY(run_scan(ctx, LoadU32{ctx->nc.as<u32>()}, N, ctx->cb.as<u64>()));
         QD_TRY(run_scan(ctx, LoadU32{ctx->wi.as<u32>()}, N, ctx->wb.as<u64>()));
-        u64 h2[2];
+        u64 *h2 = ctx->host;
         QD_HIP(hipMemcpyAsync(h2, ctx->wb.as<u64>() + N, sizeof(u64), hipMemcpyDeviceToHost, s));
         QD_HIP(hipMemcpyAsync(h2 + 1, counters + 4, sizeof(u64), hipMemcpyDeviceToHost, s));
         QD_HIP(hipStreamSynchronize(s));
@@ -3287,14 +3449,31 @@ int qd_ctx_create(qd_ctx **out, int device) {
         delete c;
         return fail(QD_ERR_HIP, std::string("hipHostMalloc: ") + hipGetErrorString(e));
     }
-    // the device address of the no-allocation scratch on this device (the
-    // device is current)
-    e = hipGetSymbolAddress(reinterpret_cast<void **>(&c->noalloc), HIP_SYMBOL(scratch));
+    e = hipHostMalloc(reinterpret_cast<void **>(&c->ring), kRing, hipHostMallocDefault);
     if (e != hipSuccess) {
         (void)hipHostFree(c->host);
         (void)hipStreamDestroy(c->stream);
         delete c;
+        return fail(QD_ERR_HIP, std::string("hipHostMalloc: ") + hipGetErrorString(e));
+    }
+    size_t freeb = 0;
+    if (hipMemGetInfo(&freeb, &c->total_mem) != hipSuccess) {
+        (void)hipGetLastError();
+        c->total_mem = 0;  // (relieve_memory then asks every time)
+    }
+    // the device address of the no-allocation scratch on this device (the
+    // device is current)
+    e = hipGetSymbolAddress(reinterpret_cast<void **>(&c->noalloc), HIP_SYMBOL(scratch));
+    if (e != hipSuccess) {
+        (void)hipHostFree(c->ring);
+        (void)hipHostFree(c->host);
+        (void)hipStreamDestroy(c->stream);
+        delete c;
         return fail(QD_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
+    }
+    {
+        std::lock_guard<std::mutex> g(g_pools_m);
+        g_pools.push_back(&c->pool);
     }
     *out = c;
     return QD_OK;
@@ -3308,7 +3487,13 @@ int qd_ctx_destroy(qd_ctx *c) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
     if (c->seggraph.exec) (void)hipGraphExecDestroy(c->seggraph.exec);
     for (DBuf *b : c->all()) b->release();
+    {
+        std::lock_guard<std::mutex> g(g_pools_m);
+        g_pools.erase(std::remove(g_pools.begin(), g_pools.end(), &c->pool), g_pools.end());
+    }
+    c->pool.trim();
     if (c->host) (void)hipHostFree(c->host);
+    if (c->ring) (void)hipHostFree(c->ring);
     for (int i = 0; i < 2 * QD_NUM_PHASES; ++i)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     (void)hipStreamDestroy(c->stream);
@@ -3343,6 +3528,7 @@ int qd_ctx_trim(qd_ctx *c) {
     QD_HIP(hipSetDevice(c->device));
     QD_HIP(hipStreamSynchronize(c->stream));
     for (DBuf *b : c->all()) b->release();
+    c->pool.trim();
     return QD_OK;
 }
 
@@ -3459,6 +3645,7 @@ int qd_state_create(qd_ctx *c, qd_state **out) {
     qd_state *s = new (std::nothrow) qd_state;
     if (!s) return fail(QD_ERR_OOM, "host allocation failed");
     s->ctx = c;
+    s->use_pool(&c->pool);
     s->objects.name = "state objects";
     s->begin.name = "state begin";
     s->size.name = "state size";
