@@ -1213,103 +1213,4 @@ __global__ __launch_bounds__(kGenThreads, kRangeWalkWaves<KIND>) void k_range_wa
     if (spill) atomicOr(err, ERR_SPILL1);
 }
 
-// Each region's entries at its running places in the buckets: bucket d
-// holds total[d] entries (every block scans the nbin totals, and the first
-// writes the nbin + 1 offsets to off), region r's first place in it is
-// bm[r * bstride + d] after the column scan.  A chunk of kPlaceChunk entries is ordered by bucket in LDS
-// first, so that consecutive lanes write consecutive places of a bucket
-// (runs of about kPlaceChunk / nbin entries) rather than one entry to each
-// of up to 64 buckets per store.
-constexpr u32 kPlaceThreads = 1024;
-constexpr u32 kPlacePer = 2;
-constexpr u32 kPlaceChunk = kPlaceThreads * kPlacePer;
-
-__global__ __launch_bounds__(kPlaceThreads) void k_region_place(const Entry *in, u64 capr, const u32 *rcount,
-                                                                u32 nreg, u32 shift, u32 nbin, const u32 *bm,
-                                                                u32 bstride, const u64 *total, u64 *off, Entry *out) {
-    // the chunk's entries by field (8-byte words: an entry's place is random,
-    // and a 32-byte store per lane to random places conflicts on the LDS
-    // banks far more than four 8-byte ones)
-    __shared__ u64 sh[kPlaceChunk], sc[kPlaceChunk];
-    __shared__ double sre[kPlaceChunk], sim[kPlaceChunk];
-    __shared__ u32 cnt[kRangeBins];
-    __shared__ u16 lst[kRangeBins];  // (16 bits: two blocks then fit a CU)
-    __shared__ u64 cur[kRangeBins];
-    __shared__ u64 tmp[kPlaceThreads / kWave + 1];
-    constexpr u32 kBinsPer = kRangeBins / kPlaceThreads;
-    static_assert(kBinsPer == 1, "a thread per bucket");
-    u64 all;
-    const u64 boff = block_excl_scan(threadIdx.x < nbin ? total[threadIdx.x] : 0, tmp, all);  // this thread's bucket's
-    if (blockIdx.x == 0) {
-        if (threadIdx.x < nbin) off[threadIdx.x] = boff;
-        if (threadIdx.x == 0) off[nbin] = all;
-    }
-    auto digit = [&](u64 key) { return nbin > 1 ? u32(key >> shift) & (nbin - 1) : 0u; };
-    for (u32 r = blockIdx.x; r < nreg; r += gridDim.x) {
-        __syncthreads();
-        if (threadIdx.x < nbin) cur[threadIdx.x] = boff + bm[u64(r) * bstride + threadIdx.x];
-        const u32 n = rcount[r];
-        const Entry *src = in + u64(r) * capr;
-        for (u32 c0 = 0; c0 < n; c0 += kPlaceChunk) {
-            const u32 m = min(kPlaceChunk, n - c0);
-            __syncthreads();  // the previous chunk is written and its counts added
-            for (u32 i = threadIdx.x; i < nbin; i += kPlaceThreads) cnt[i] = 0;
-            __syncthreads();
-            Entry e[kPlacePer];
-            u32 dr[kPlacePer];
-#pragma unroll
-            for (u32 q = 0; q < kPlacePer; ++q) {
-                const u32 j = threadIdx.x + kPlaceThreads * q;
-                if (j < m) {
-                    e[q] = src[c0 + j];
-                    const u32 d = digit(e[q].hash);
-                    dr[q] = (d << 16) | atomicAdd(&cnt[d], 1u);
-                }
-            }
-            __syncthreads();
-            // the buckets' starts within the chunk: an exclusive scan of cnt
-            u32 v[kBinsPer];
-            u64 sum = 0;
-#pragma unroll
-            for (u32 q = 0; q < kBinsPer; ++q) {
-                const u32 b = threadIdx.x * kBinsPer + q;
-                v[q] = b < nbin ? cnt[b] : 0u;
-                sum += v[q];
-            }
-            u64 tot;
-            u64 run = block_excl_scan(sum, tmp, tot);
-#pragma unroll
-            for (u32 q = 0; q < kBinsPer; ++q) {
-                const u32 b = threadIdx.x * kBinsPer + q;
-                if (b < nbin) lst[b] = u16(run);
-                run += v[q];
-            }
-            __syncthreads();
-#pragma unroll
-            for (u32 q = 0; q < kPlacePer; ++q) {
-                const u32 j = threadIdx.x + kPlaceThreads * q;
-                if (j < m) {
-                    const u32 at = lst[dr[q] >> 16] + (dr[q] & 0xFFFF);
-                    sh[at] = e[q].hash;
-                    sc[at] = e[q].cand;
-                    sre[at] = e[q].re;
-                    sim[at] = e[q].im;
-                }
-            }
-            __syncthreads();
-            for (u32 j = threadIdx.x; j < m; j += kPlaceThreads) {
-                Entry x;
-                x.hash = sh[j];
-                x.cand = sc[j];
-                x.re = sre[j];
-                x.im = sim[j];
-                const u32 d = digit(x.hash);
-                out[cur[d] + (j - lst[d])] = x;
-            }
-            __syncthreads();
-            for (u32 i = threadIdx.x; i < nbin; i += kPlaceThreads) cur[i] += cnt[i];
-        }
-    }
-}
-
 }  // namespace qd

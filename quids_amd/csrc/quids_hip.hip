@@ -90,6 +90,8 @@ static int fail(int code, const std::string &msg) {
 // device buffers
 // ===========================================================================
 constexpr size_t kBigAlloc = 48ull << 30;
+// Workgroups of the second radix pass, at most: two a CU.
+constexpr unsigned kL2Grid = 512;
 
 static double dbuf_ms();
 static void dbuf_log(const char *what, size_t bytes, double ms, const char *name = nullptr);
@@ -963,6 +965,29 @@ static int dedup_phase(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *woff
     return QD_OK;
 }
 
+// The second radix pass over nbk1 first-level buckets of `in` into cap2-entry
+// sub-buckets of E2 (k_level2_runs): counts to cnt2, the entries beyond to the
+// overflow list.  The context's counters 4 and 7 must be zero; with parts
+// beyond 1 (workgroups per bucket), so must cnt2.
+static int level2(qd_ctx *ctx, const Entry *in, u64 in_stride, const u64 *off1, u64 nbk1, u32 b1, u32 b2, u64 cap2,
+                  Entry *E2, u32 parts) {
+    u64 *counters = ctx->counters.as<u64>();
+    u32 *errw = reinterpret_cast<u32 *>(counters + 4);
+    auto launch = [&](auto kern, u64 grid) {
+        hipLaunchKernelGGL(kern, dim3(unsigned(grid)), dim3(1024), 0, ctx->stream, in, in_stride, off1, nbk1, b1, b2,
+                           cap2, E2, ctx->cnt2.as<u64>(), errw, ctx->ovf.as<Entry>(), counters + 7, parts,
+                           (LeanPlan *)nullptr);
+    };
+    if (b2 <= kSplitBits) launch(k_level2_runs<kSplitBits>, parts > 1 ? nbk1 * parts : std::min<u64>(nbk1, kL2Grid));
+    else if (b2 <= kSplitWideBits) launch(k_level2_runs<kSplitWideBits>, std::min<u64>(nbk1, kL2Grid));
+    else
+        hipLaunchKernelGGL(k_level2_fixed, dim3(unsigned(std::min<u64>(nbk1, 128))), dim3(1024), 0, ctx->stream, in,
+                           in_stride, off1, nbk1, b1, b2, cap2, E2, ctx->cnt2.as<u64>(), errw, ctx->ovf.as<Entry>(),
+                           counters + 7, (LeanPlan *)nullptr);
+    QD_HIP(hipGetLastError());
+    return QD_OK;
+}
+
 // Partition (one or two radix passes on the top key bits) and dedup of n
 // candidates with keys H0 and magnitudes M0 (CI: candidate index of each
 // position, null when the position is the candidate index).  hist1 holds the
@@ -1035,16 +1060,7 @@ static int partition_dedup(qd_ctx *ctx, const u64 *H0, const double2 *M0, const 
         Entry *E2 = ctx->ebuf2.as<Entry>();
         u32 ew = ERR_SPILL;
         if (fixed) {
-            // one workgroup per first-level bucket, on at most half the CUs
-            // at a time: the open lines of the sub-buckets (2^b2 per
-            // workgroup) then fit L2 better, and the pass runs faster than
-            // on every CU
-            int ncu2 = 256;
-            (void)hipDeviceGetAttribute(&ncu2, hipDeviceAttributeMultiprocessorCount, ctx->device);
-            const unsigned g2 = unsigned(std::min<u64>(nb1, std::max(ncu2 / 2, 1)));
-            hipLaunchKernelGGL(k_level2_fixed, dim3(g2), dim3(1024), 0, s, (const Entry *)E1, in_stride,
-                               ctx->off1.as<u64>(), nb1, b1, b2, cap2, E2, ctx->cnt2.as<u64>(), errw, ctx->ovf.as<Entry>(), counters + 7, (LeanPlan *)nullptr);
-            QD_HIP(hipGetLastError());
+            QD_TRY(level2(ctx, E1, in_stride, ctx->off1.as<u64>(), nb1, b1, b2, cap2, E2, 1));
             QD_TRY(run_scan(ctx, LoadU64{ctx->cnt2.as<u64>()}, nb, ctx->off2.as<u64>()));
             QD_TRY(sync_read(ctx, errw, sizeof(u32), &ew));
             rstride = cap2;
@@ -1731,6 +1747,12 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
     QD_TRY(carve(ctx->rpart[0], std::max<u64>(u64(ngroups) * gbytes, nmax * sizeof(Entry))));
     std::vector<u32> rc(u64(ngroups) * gr);
     bool l2_exact = false;  // second pass with exact offsets (after a spill)
+    // A group has at most 128 first-level buckets (nb1 / 8): several
+    // workgroups each, which take their places in a sub-bucket from one
+    // counter (one workgroup each left half the CUs idle: 152 us a group of
+    // 7.3e6 candidates, now 107); beyond 2^8 sub-buckets a chunk would go to
+    // memory for a place of every few entries.
+    const u32 l2_parts = b2 && b2 <= 8 ? u32(std::max<u64>(kL2Grid / gbk, 1)) : 1;
     tl[4] = wall_ms();
     phase_mark(ctx, PH_COLL_INSERT);
     for (const Pass &pass : passes) {
@@ -1834,9 +1856,10 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
                 const u32 *rcg = ctx->rcnt.as<u32>() + u64(g) * gr;
                 prof_begin(ctx, QD_PHASE_PARTITION);
                 const u64 g0 = u64(g) * gbk;  // the group's first bucket: its columns of bmat
-                hipLaunchKernelGGL(k_region_place, dim3(gr), dim3(kPlaceThreads), 0, s, (const Entry *)GB.g[g], capr,
+                hipLaunchKernelGGL(k_region_place, dim3(gr), dim3(kSplitThreads), 0, s, (const Entry *)GB.g[g], capr,
                                    rcg, u32(gr), 64 - b1, u32(gbk), (const u32 *)ctx->bmat.as<u32>() + g0, u32(nb1),
-                                   (const u64 *)ctx->cur1.as<u64>() + g0, ctx->off1.as<u64>(), ctx->abuf.as<Entry>());
+                                   (const u64 *)ctx->cur1.as<u64>() + g0, ctx->off1.as<u64>(), ctx->abuf.as<Entry>(),
+                                   l2_parts > 1 ? ctx->cnt2.as<u64>() : nullptr, l2_parts > 1 ? nb2g : 0);
                 QD_HIP(hipGetLastError());
                 prof_end(ctx, QD_PHASE_PARTITION);
                 gin = ctx->abuf.as<Entry>();
@@ -1864,13 +1887,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
                 const bool exact = l2_exact;
                 prof_begin(ctx, QD_PHASE_PARTITION);
                 if (b2 && !exact) {
-                    int ncu2 = 256;
-                    (void)hipDeviceGetAttribute(&ncu2, hipDeviceAttributeMultiprocessorCount, ctx->device);
-                    const unsigned g2 = unsigned(std::min<u64>(gbk, std::max(ncu2 / 2, 1)));
-                    hipLaunchKernelGGL(k_level2_fixed, dim3(g2), dim3(1024), 0, s, gin, u64(0), go, gbk, b1, b2, cap2,
-                                       E2, ctx->cnt2.as<u64>(), errw, ctx->ovf.as<Entry>(), counters + 7,
-                                       (LeanPlan *)nullptr);
-                    QD_HIP(hipGetLastError());
+                    QD_TRY(level2(ctx, gin, 0, go, gbk, b1, b2, cap2, E2, single ? l2_parts : 1));
                     QD_TRY(run_scan(ctx, LoadU64{ctx->cnt2.as<u64>()}, nb2g, ctx->off2.as<u64>()));
                     rstride = cap2;
                     if (!single) {  // (the uniques will overwrite gin: look before the dedup)
@@ -2314,8 +2331,9 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
     prof_end(ctx, QD_PHASE_GENERATE);
     prof_begin(ctx, QD_PHASE_PARTITION);
     if (two)
-        hipLaunchKernelGGL(k_level2_fixed, dim3(128), dim3(1024), 0, s, (const Entry *)E1, u64(0), (const u64 *)cnt1,
-                           u64(0), 0u, 0u, u64(0), E2, cnt2, (u32 *)nullptr, (Entry *)nullptr, (u64 *)nullptr, lp);
+        hipLaunchKernelGGL(k_level2_runs<kSplitBits>, dim3(kL2Grid), dim3(1024), 0, s, (const Entry *)E1, u64(0),
+                           (const u64 *)cnt1, u64(0), 0u, 0u, u64(0), E2, cnt2, (u32 *)nullptr, (Entry *)nullptr,
+                           (u64 *)nullptr, 1u, lp);
     hipLaunchKernelGGL(k_lean_bscan, dim3(1), dim3(1024), 0, s, (const u64 *)cnt1, (const u64 *)cnt2,
                        (const LeanPlan *)lp, ctx->off2.as<u64>());
     QD_HIP(hipGetLastError());
