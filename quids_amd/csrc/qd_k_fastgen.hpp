@@ -333,83 +333,74 @@ using Walk = WalkT<cplx>;
 // w.d on entry (`bits` a u32, or a u64 for a walk over more than 32
 // decisions at once); returns when the next decision is not available or
 // the walk is complete.
-template <typename W, typename KC, typename BT>
-__device__ inline void sm_run(W &w, const PDesc &pd, const u64 *tab, BT bits, u32 dlimit, const KC &k) {
+//
+// The cases of a node share one emission (and a taken split a second), with
+// its table slot and sides selected: lanes of one wavefront walk several
+// parents, whose nodes differ, and each case's own code ran in turn; and the
+// walk is inlined 15 times in a generate.  START: the walk may be at its
+// first node; ONE: at most one decision is available, with the bit `bits`.
+template <typename KC>
+__device__ __attribute__((always_inline)) inline void mul_factor(cplx &mag, const KC &k, bool take, bool merge) {
+    const cplx a = merge ? k.dc : k.d, b = merge ? cneg(k.dnc) : k.dn;
+    mag = cmul(mag, take ? a : b);
+}
+template <typename M, typename KC>
+__device__ __attribute__((always_inline)) inline void mul_factor(M &mag, const KC &k, bool take, bool merge) {
+    if (take) mag = merge ? cmul(mag, k.dc) : cmul(mag, k.d);
+    else mag = merge ? cmul(mag, cneg(k.dnc)) : cmul(mag, k.dn);
+}
+
+template <bool START = true, bool ONE = false, typename W, typename KC, typename BT>
+__device__ __attribute__((always_inline)) inline void sm_run(W &w, const PDesc &pd, const u64 *tab, BT bits, u32 dlimit,
+                                                             const KC &k) {
     const u32 n = pd.n;
     const u32 d0 = w.d;
-    auto emit = [&](u64 root, bool l, bool r) {
+    auto bit = [&]() -> bool { return ONE ? bits & 1 : (bits >> (w.d - d0)) & 1; };
+    auto emit = [&](u64 root, bool l, bool r) __attribute__((always_inline)) {
         w.nh = step_pm(w.nh, root);
         if (l) w.lh = small_step_pm(w.lh, w.c);
         if (r) w.rh = small_step_pm(w.rh, w.c);
         ++w.c;
     };
-    if (!w.started) {
-        if (pd.flags & PD_LM) {
+    if (START && !w.started) {
+        // the last node merging with the first (LM), or the first node's
+        // split (FS), is the first decision
+        const bool lm = pd.flags & PD_LM, fs = pd.flags & PD_FS;
+        bool first = false;  // the first node is done with
+        w.end = n;
+        if (lm || fs) {
             if (w.d >= dlimit) return;
-            const bool take = (bits >> (w.d++ - d0)) & 1;
-            if (take) {
-                w.mag = cmul(w.mag, k.dc);
-                emit(tab[kSmSlots * (n - 1) + 1], true, true);
-                w.i = 1;
-                w.end = n - 1;
-            } else {
-                w.mag = cmul(w.mag, cneg(k.dnc));
-                w.i = 0;
-                w.end = n;
+            const bool take = bit(), whole = pd.flags & PD_HMLZ;
+            ++w.d;
+            mul_factor(w.mag, k, take, lm);
+            first = take || fs;
+            if (first) {
+                // a merge; the node unsplit; its left half; its right half,
+                // with the left one going last
+                emit(tab[lm ? kSmSlots * (n - 1) + 1 : !take ? 0u : whole ? 1u : 2u], lm || !take || whole,
+                     lm || !take || !whole);
+                if (fs && take && whole) emit(tab[2], false, true);
             }
-        } else if (pd.flags & PD_FS) {
-            if (w.d >= dlimit) return;
-            const bool take = (bits >> (w.d++ - d0)) & 1;
-            if (take) {
-                w.mag = cmul(w.mag, k.d);
-                if (pd.flags & PD_HMLZ) {
-                    emit(tab[1], true, false);
-                    emit(tab[2], false, true);
-                } else {
-                    w.overflow = true;
-                    emit(tab[2], false, true);
-                }
-            } else {
-                w.mag = cmul(w.mag, k.dn);
-                emit(tab[0], true, true);
-            }
-            w.i = 1;
-            w.end = n;
-        } else {
-            w.i = 0;
-            w.end = n;
+            w.overflow = fs && take && !whole;
+            w.end = lm && take ? n - 1 : n;
         }
+        w.i = first ? 1 : 0;
         w.started = true;
     }
     while (w.i < w.end) {
         const u32 i = w.i;
-        const bool l = (pd.lmask >> i) & 1, r = (pd.rmask >> i) & 1;
+        const bool l = (pd.lmask >> i) & 1, r = (pd.rmask >> i) & 1, split = l && r;
+        bool take = false;
         if ((pd.dmask >> i) & 1) {
             if (w.d >= dlimit) return;
-            const bool take = (bits >> (w.d++ - d0)) & 1;
-            if (l && r) {  // split
-                if (take) {
-                    w.mag = cmul(w.mag, k.d);
-                    emit(tab[kSmSlots * i + 1], true, false);
-                    emit(tab[kSmSlots * i + 2], false, true);
-                } else {
-                    w.mag = cmul(w.mag, k.dn);
-                    emit(tab[kSmSlots * i], l, r);
-                }
-            } else {  // merge with node i+1 (which carries no decision)
-                if (take) {
-                    w.mag = cmul(w.mag, k.dc);
-                    emit(tab[kSmSlots * i + 1], true, true);
-                    ++w.i;
-                } else {
-                    w.mag = cmul(w.mag, cneg(k.dnc));
-                    emit(tab[kSmSlots * i], l, r);
-                }
-            }
-        } else {
-            emit(tab[kSmSlots * i], l, r);
+            take = bit();
+            ++w.d;
+            mul_factor(w.mag, k, take, !split);
         }
-        ++w.i;
+        // (a taken merge is with node i + 1, which carries no decision)
+        emit(tab[kSmSlots * i + (take ? 1u : 0u)], l || take, take ? !split : r);
+        if (take && split) emit(tab[kSmSlots * i + 2], false, true);
+        w.i += take && !split ? 2 : 1;
     }
 }
 
@@ -585,10 +576,10 @@ __device__ inline u64 flip_child(const PDesc &pd, u64 bits, const cplx *ct, cplx
 // runs once per child, u a compile-time constant after unrolling.
 static_assert(kItemBits == 3, "walk_item enumerates three decision levels");
 
-template <int KIND, typename W, typename KC>
+template <int KIND, bool START = true, bool ONE = false, typename W, typename KC>
 __device__ __attribute__((always_inline)) inline void walk_step(W &w, const PDesc &pd, const u64 *ptab, u32 bit,
                                                                 u32 dlimit, const KC &k) {
-    if (KIND == QD_RULE_QCGD_SPLIT_MERGE) sm_run(w, pd, ptab, bit, dlimit, k);
+    if (KIND == QD_RULE_QCGD_SPLIT_MERGE) sm_run<START, ONE>(w, pd, ptab, bit, dlimit, k);
     else flip_run<KIND == QD_RULE_QCGD_COIN>(w, pd, bit, dlimit, k);
 }
 
@@ -599,17 +590,17 @@ __device__ __attribute__((always_inline)) inline void walk_item(const W &pre, co
     for (u32 b0 = 0; b0 < 2; ++b0) {
         if (b0 && t < 1) break;
         W w0 = pre;
-        walk_step<KIND>(w0, pd, ptab, b0, s + 1, k);
+        walk_step<KIND, true, true>(w0, pd, ptab, b0, s + 1, k);
 #pragma unroll
         for (u32 b1 = 0; b1 < 2; ++b1) {
             if (b1 && t < 2) break;
             W w1 = w0;
-            walk_step<KIND>(w1, pd, ptab, b1, s + 2, k);
+            walk_step<KIND, false, true>(w1, pd, ptab, b1, s + 2, k);
 #pragma unroll
             for (u32 b2 = 0; b2 < 2; ++b2) {
                 if (b2 && t < 3) break;
                 W w2 = w1;
-                walk_step<KIND>(w2, pd, ptab, b2, s + 3, k);
+                walk_step<KIND, false, true>(w2, pd, ptab, b2, s + 3, k);
                 u64 h;
                 if (KIND == QD_RULE_QCGD_SPLIT_MERGE) h = sm_finish(w2, ptab);
                 else h = finish_pm(pd.nf, w2.lh, w2.rh);
@@ -620,6 +611,51 @@ __device__ __attribute__((always_inline)) inline void walk_item(const W &pre, co
 }
 
 constexpr int kGenThreads = 256;
+
+// The split_merge tables of the parents of one chunk of kGenThreads work
+// items (a dozen or two: 20 items share a parent of 12 nodes), staged in LDS:
+// every node of a walk reads its root hash there, 64 lanes at 3-4 parents'
+// places, which from memory cost the generate of a 12-node step more issue
+// slots than its arithmetic.
+template <u32 CAP>
+struct SmStage {
+    u64 t[CAP];
+    u64 base[kGenThreads];  // the parents' tables in tab
+    u8 n[kGenThreads];      // their node counts
+    u32 maxn[kGenThreads / kWave];
+};
+
+// Stages the tables of the chunk's parents pf, pf + 1, ... (swb: wb of the
+// first kGenThreads + 1 of them) if they fit; returns the 8-byte words between
+// two parents' tables in S.t, or 0.  wend: the chunk's first item beyond.
+// Called by the whole workgroup, with swb in place; its last barrier
+// publishes the tables.
+template <u32 CAP>
+__device__ inline u32 stage_tables(SmStage<CAP> &S, const PDesc *D, const u64 *tab, const u64 *pbegin, u64 pf,
+                                   const u64 *swb, u64 wend) {
+    const u32 t = threadIdx.x;
+    const u32 np = u32(__syncthreads_count(swb[t] < wend));
+    u32 n = 0;
+    if (t < np) {
+        n = D[pf + t].n;
+        S.base[t] = sm_tab_base(pbegin[pf + t]);
+        S.n[t] = u8(n);
+    }
+#pragma unroll
+    for (int o = kWave / 2; o; o >>= 1) n = max(n, u32(__shfl_xor(int(n), o, kWave)));
+    if ((t & (kWave - 1)) == 0) S.maxn[t / kWave] = n;
+    __syncthreads();
+#pragma unroll
+    for (u32 w = 0; w < kGenThreads / kWave; ++w) n = max(n, S.maxn[w]);
+    const u32 stride = (kSmSlots * n) | 1u;  // (odd: parents start on different banks)
+    if (np * stride > CAP || swb[np] < wend) return 0;
+    for (u32 i = t; i < np * stride; i += kGenThreads) {
+        const u32 q = i / stride, r = i - q * stride;
+        if (r < kSmSlots * S.n[q]) S.t[i] = tab[S.base[q] + r];
+    }
+    __syncthreads();
+    return stride;
+}
 
 // Parent of the first work item of every chunk of kGenThreads items (the
 // chunk a generate workgroup takes per iteration): cpar[c] = the last p
@@ -710,14 +746,29 @@ __global__ __launch_bounds__(kGenThreads) void k_generate_fast(const PDesc *D, c
 // ---------------------------------------------------------------------------
 // Generate fused with the first radix pass (at most 2^9 buckets): a block
 // ranks its children per bucket of the top b1 key bits in LDS, reserves one
-// range per bucket and writes 32-byte entries {key, candidate, magnitude}
-// into fixed-capacity buckets (bucket d owns [d * cap1, (d + 1) * cap1) of
-// E1; cnt1[d] counts them).  A bucket that would pass cap1 drops the excess
-// and raises ERR_SPILL1: the step then redoes generate and partition the
-// two-kernel way.  BATCH as in k_generate_fast.
+// range per bucket, orders the children by bucket in LDS and writes them as
+// 32-byte entries {key, candidate, magnitude}, in runs, into fixed-capacity
+// buckets (bucket d owns [d * cap1, (d + 1) * cap1) of E1; cnt1[d] counts
+// them).  A bucket that would pass cap1 drops the excess and raises
+// ERR_SPILL1: the step then redoes generate and partition the two-kernel way.
+// BATCH as in k_generate_fast.
+//
+// Bound by the walks' arithmetic (64-bit multiplications, a tree of 14
+// segments per item) for split_merge, by the entries' writes for the flip
+// rules.  3.3e8 split_merge children of 12 nodes 7.5 ms (13.3 ms with a case
+// per kind of node, the tables in memory and each lane writing its entries
+// where they belong: 10.1 with the tables staged, 9.3 with one emission for
+// all cases, 7.5 with runs); 2.7e8 erase_create children 3.9 ms (6.3 ms).
 // ---------------------------------------------------------------------------
 constexpr u32 ERR_SPILL1 = 32u;
 constexpr u32 kFusedBins = 512;
+
+// A window of a workgroup's children in bucket order.
+template <u32 WINDOW>
+struct GenRuns {
+    u64 key[WINDOW], cand[WINDOW];
+    double re[WINDOW], im[WINDOW];
+};
 
 template <int KIND, bool BATCH>
 __global__ __launch_bounds__(kGenThreads, 3) void k_generate_scatter(const PDesc *D, const double2 *pmag, const u64 *cb,
@@ -728,14 +779,21 @@ __global__ __launch_bounds__(kGenThreads, 3) void k_generate_scatter(const PDesc
                                                                  u64 fold) {
     constexpr u32 kKids = 1u << kItemBits;
     __shared__ u32 bcnt[kFusedBins];
-    __shared__ u64 bbase[kFusedBins];  // first reserved slot of the bucket
-    __shared__ u64 bidx[kFusedBins];   // its entry index in E1: bucket * cap1 + first slot
+    __shared__ u16 lst[kFusedBins];   // first place of the bucket within the ordered children
+    __shared__ u64 bidx[kFusedBins];  // entry index in E1 of its first reserved slot, less lst
+    __shared__ u32 wtot[kGenThreads / kWave];
     __shared__ u64 swb[kGenThreads + 1];
     __shared__ u64 pfirst;
     // batched: the children's magnitudes wait in LDS (each thread its own
     // slots) rather than registers, which the instance search and offsets
     // need
     __shared__ double2 sms[BATCH ? kKids * kGenThreads : 1];
+    // (three workgroups fit a CU by registers: 53 KB each)
+    constexpr bool kSm = KIND == QD_RULE_QCGD_SPLIT_MERGE;
+    __shared__ union {
+        SmStage<kSm ? (BATCH ? 640 : 2048) : 1> stage;  // during the walks
+        GenRuns<BATCH ? 1 : 1024> runs;
+    } sh;
     const u32 nbin = 1u << b1;
     QcgdCoef k = coef_of(rule);
     bool spill = false;
@@ -746,7 +804,13 @@ __global__ __launch_bounds__(kGenThreads, 3) void k_generate_scatter(const PDesc
         __syncthreads();
         const u64 pf = pfirst;
         for (u32 q = threadIdx.x; q <= kGenThreads; q += blockDim.x) swb[q] = pf + q <= N ? wb[pf + q] : ~0ull;
-        __syncthreads();
+        u32 stride = 0;
+        if constexpr (kSm) {
+            __syncthreads();
+            stride = stage_tables(sh.stage, D, tab, pbegin, pf, swb, min(w0 + kGenThreads, W));
+        } else {
+            __syncthreads();
+        }
         const u64 w = w0 + threadIdx.x;
         // children u < nk of this item; the arrays are indexed by the
         // unrolled loop counter only, so they stay in registers
@@ -787,41 +851,87 @@ __global__ __launch_bounds__(kGenThreads, 3) void k_generate_scatter(const PDesc
             const double2 m0 = pmag[p];
             Walk pre{};
             pre.mag = cplx{m0.x, m0.y};
-            const u64 *ptab = tab + sm_tab_base(pbegin[p]);
-            if (KIND == QD_RULE_QCGD_SPLIT_MERGE) sm_run(pre, pd, ptab, j0, s, k);
-            else flip_run<KIND == QD_RULE_QCGD_COIN>(pre, pd, j0, s, k);
             cbase = cb[p] + j0;
-            walk_item<KIND>(pre, pd, ptab, s, t, k, [&](u32 u, u64 h, const cplx &m) {
-                if (BATCH) h += hadd;
-                const u32 d = b1 ? u32(h >> (64 - b1)) : 0u;
-                hs[u] = h;
-                if (BATCH) sms[u * kGenThreads + threadIdx.x] = make_double2(m.re, m.im);
-                else ms[u] = make_double2(m.re, m.im);
-                br[u] = (d << 16) | atomicAdd(&bcnt[d], 1u);
-            });
+            auto walk = [&](const u64 *ptab) __attribute__((always_inline)) {
+                walk_step<KIND>(pre, pd, ptab, j0, s, k);
+                walk_item<KIND>(pre, pd, ptab, s, t, k, [&](u32 u, u64 h, const cplx &m) {
+                    if (BATCH) h += hadd;
+                    const u32 d = b1 ? u32(h >> (64 - b1)) : 0u;
+                    hs[u] = h;
+                    if (BATCH) sms[u * kGenThreads + threadIdx.x] = make_double2(m.re, m.im);
+                    else ms[u] = make_double2(m.re, m.im);
+                    br[u] = (d << 16) | atomicAdd(&bcnt[d], 1u);
+                });
+            };
+            if (kSm && stride) walk(sh.stage.t + u32(p - pf) * stride);
+            else walk(tab + sm_tab_base(pbegin[p]));
         }
         __syncthreads();
-        for (u32 i = threadIdx.x; i < nbin; i += blockDim.x)
-            if (bcnt[i]) {
-                const u64 b0 = atomicAdd(reinterpret_cast<unsigned long long *>(cnt1 + i), (unsigned long long)bcnt[i]);
-                bbase[i] = b0;
-                bidx[i] = u64(i) * cap1 + b0;
-            }
-        __syncthreads();
+        // the buckets' places: first within the ordered children, then in E1
+        // (neighbouring lanes on neighbouring counters: their atomics share
+        // a request)
+        u32 total = 0;
+        for (u32 d0 = 0; d0 < nbin; d0 += kGenThreads) {
+            const u32 d = d0 + threadIdx.x, v = d < nbin ? bcnt[d] : 0u;
+            u64 b0 = 0;
+            if (v) b0 = atomicAdd(reinterpret_cast<unsigned long long *>(cnt1 + d), (unsigned long long)v);
+            u32 run = v;
 #pragma unroll
-        for (u32 u = 0; u < kKids; ++u) {
-            if (u < nk) {
-                const u32 d = br[u] >> 16, r = br[u] & 0xFFFF;
-                if (bbase[d] + r < cap1) {
-                    const double2 mu = BATCH ? sms[u * kGenThreads + threadIdx.x] : ms[u];
-                    Entry e;
-                    e.hash = hs[u];
-                    e.cand = cbase + (u64(u) << s);
-                    e.re = mu.x;
-                    e.im = mu.y;
-                    E1[bidx[d] + r] = e;
-                } else {
-                    spill = true;
+            for (int o = 1; o < kWave; o <<= 1) {
+                const u32 up = __shfl_up(run, o, kWave);
+                if ((threadIdx.x & (kWave - 1)) >= u32(o)) run += up;
+            }
+            if (d0) __syncthreads();
+            if ((threadIdx.x & (kWave - 1)) == kWave - 1) wtot[threadIdx.x / kWave] = run;
+            __syncthreads();
+            run += total - v;
+#pragma unroll
+            for (u32 x = 0; x < kGenThreads / kWave; ++x) {
+                if (x < threadIdx.x / kWave) run += wtot[x];
+                total += wtot[x];
+            }
+            if (v) {
+                lst[d] = u16(run);
+                bidx[d] = u64(d) * cap1 + b0 - run;
+            }
+        }
+        __syncthreads();
+        if constexpr (BATCH) {  // (no LDS left for runs at three workgroups a CU)
+#pragma unroll
+            for (u32 u = 0; u < kKids; ++u) {
+                if (u < nk) {
+                    const u32 d = br[u] >> 16;
+                    const u64 at = bidx[d] + lst[d] + (br[u] & 0xFFFF);
+                    const double2 mu = sms[u * kGenThreads + threadIdx.x];
+                    if (at < u64(d + 1) * cap1) E1[at] = Entry{hs[u], cbase + (u64(u) << s), mu.x, mu.y};
+                    else spill = true;
+                }
+            }
+        } else {
+            // written in runs, a window of the ordered children at a time
+            constexpr u32 kWindow = 1024;
+            for (u32 first = 0; first < total; first += kWindow) {
+                if (first) __syncthreads();
+#pragma unroll
+                for (u32 u = 0; u < kKids; ++u) {
+                    if (u < nk) {
+                        const u32 at = lst[br[u] >> 16] + (br[u] & 0xFFFF) - first;
+                        if (at < kWindow) {
+                            sh.runs.key[at] = hs[u];
+                            sh.runs.cand[at] = cbase + (u64(u) << s);
+                            sh.runs.re[at] = ms[u].x;
+                            sh.runs.im[at] = ms[u].y;
+                        }
+                    }
+                }
+                __syncthreads();
+                const u32 m = min(total - first, kWindow);
+                for (u32 j = threadIdx.x; j < m; j += kGenThreads) {
+                    const Entry e{sh.runs.key[j], sh.runs.cand[j], sh.runs.re[j], sh.runs.im[j]};
+                    const u32 d = b1 ? u32(e.hash >> (64 - b1)) : 0u;
+                    const u64 at = bidx[d] + first + j;
+                    if (at < u64(d + 1) * cap1) E1[at] = e;
+                    else spill = true;
                 }
             }
         }
@@ -855,6 +965,8 @@ __global__ __launch_bounds__(kGenThreads) void k_range_count(const PDesc *D, con
     __shared__ u32 lh[kHistBins];
     __shared__ u64 swb[kGenThreads + 1];
     __shared__ u64 pfirst;
+    constexpr bool kSm = KIND == QD_RULE_QCGD_SPLIT_MERGE;
+    __shared__ SmStage<kSm ? 2048 : 1> stage;
     for (int i = threadIdx.x; i < kHistBins; i += blockDim.x) lh[i] = 0;
     const QcgdCoef k = coef_of(rule);
     const u32 S = (1u << T) - 1;
@@ -865,6 +977,8 @@ __global__ __launch_bounds__(kGenThreads) void k_range_count(const PDesc *D, con
         const u64 pf = pfirst;
         for (u32 q = threadIdx.x; q <= kGenThreads; q += blockDim.x) swb[q] = pf + q <= N ? wb[pf + q] : ~0ull;
         __syncthreads();
+        u32 stride = 0;
+        if constexpr (kSm) stride = stage_tables(stage, D, tab, pbegin, pf, swb, min(w0 + kGenThreads, W));
         const u64 w = w0 + threadIdx.x;
         if (w >= W) continue;
         u64 p;
@@ -886,17 +1000,19 @@ __global__ __launch_bounds__(kGenThreads) void k_range_count(const PDesc *D, con
         const double2 m0 = pmag[p];
         Walk pre{};
         pre.mag = cplx{m0.x, m0.y};
-        const u64 *ptab = tab + sm_tab_base(pbegin[p]);
-        if (KIND == QD_RULE_QCGD_SPLIT_MERGE) sm_run(pre, pd, ptab, j0, s, k);
-        else flip_run<KIND == QD_RULE_QCGD_COIN>(pre, pd, j0, s, k);
         u32 tg[1u << kItemBits];
 #pragma unroll
         for (u32 u = 0; u < (1u << kItemBits); ++u) tg[u] = S;
-        walk_item<KIND>(pre, pd, ptab, s, t, k, [&](u32 u, u64 h, const cplx &) {
-            const u32 bin = u32(h >> 52);
-            atomicAdd(&lh[bin], 1u);
-            tg[u] = (bin * S) >> 12;
-        });
+        auto walk = [&](const u64 *ptab) __attribute__((always_inline)) {
+            walk_step<KIND>(pre, pd, ptab, j0, s, k);
+            walk_item<KIND>(pre, pd, ptab, s, t, k, [&](u32 u, u64 h, const cplx &) {
+                const u32 bin = u32(h >> 52);
+                atomicAdd(&lh[bin], 1u);
+                tg[u] = (bin * S) >> 12;
+            });
+        };
+        if (kSm && stride) walk(stage.t + u32(p - pf) * stride);
+        else walk(tab + sm_tab_base(pbegin[p]));
 #pragma unroll
         for (u32 b = 0; b < kMaxTagBits; ++b) {
             if (b >= T) break;
