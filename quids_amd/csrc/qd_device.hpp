@@ -69,6 +69,10 @@ __device__ inline u64 block_excl_scan(u64 v, u64 *tmp, u64 &total) {
     return r;
 }
 
+// An error word that may lie in pinned host memory (a modifier's: it raises
+// one code only, so a store does).
+__device__ inline void raise_error(u32 *err, u32 code) { *reinterpret_cast<volatile u32 *>(err) = code; }
+
 // ---------------------------------------------------------------------------
 // A step driven from the device (qd_k_lean.hpp): its sizes and layout, read
 // by each kernel when it starts.
@@ -94,7 +98,7 @@ struct LeanPlan {
     u64 K, bytes;      // survivors and their padded bytes
     u32 b1, b2;        // bits of the radix passes
     u32 d1;            // select: the first digit
-    u32 ticket[3];     // next tiles of the look-back kernels
+    u32 ticket[3];     // next tiles of the look-back kernels; blocks of the generate that ended
     u32 stop[LEAN_EMIT];  // LEAN_* by kernel (the dedup's: counters 5 and 6)
 };
 // What the last kernel reports to the host (pinned memory).

@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void k_modifier_adjoint(const u8 *obj, const u
                                                           qd_modifier m, double2 *g, u32 *err) {
     for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < N; i += u64(gridDim.x) * blockDim.x) {
         if ((m.kind == QD_MOD_YGATE || m.kind == QD_MOD_ZGATE) && m.bit >= size[i]) {
-            atomicOr(err, ERR_BIT);
+            raise_error(err, ERR_BIT);
             continue;
         }
         const cplx f = modifier_factor_after(m, obj + begin[i]);

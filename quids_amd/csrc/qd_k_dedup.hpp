@@ -368,7 +368,8 @@ constexpr int kWideCandBits = 40;
 template <int T, int CAP, int TS>
 __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const u64 *woff, u64 nbk, u32 L, double tol,
                                              u64 *UH, u64 *UR, double2 *UM, u32 *UK, u64 *counters, u64 *nhist,
-                                             u64 *biglist, u64 *redolist, LeanPlan *lp, const Entry *E2) {
+                                             u64 *biglist, u64 *redolist, LeanPlan *lp, const Entry *E2,
+                                             u32 *slotof) {
     if (lp) {  // a step driven from the device: the buckets of E, or of E2 after a second pass
         if (lean_stopped(lp, LEAN_DEDUP)) return;
         L = lp->b1 + lp->b2;
@@ -661,6 +662,7 @@ __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const 
                 UR[pos] = rc[k];
                 UM[pos] = rs[k];
                 if (UK) UK[pos] = nk[k];
+                if (slotof) slotof[rc[k]] = u32(pos);  // (driven from the device: every unique survives)
             }
             run += u32(__popcll(km[k]));
         }

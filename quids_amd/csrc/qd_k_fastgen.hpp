@@ -269,7 +269,7 @@ __device__ inline void step_object(u8 *obj, const u64 *begin, const u32 *size, u
         }
     }
     if (!valid) {
-        if (sl == 0) atomicOr(err, ERR_OBJECT);
+        if (sl == 0) raise_error(err, ERR_OBJECT);
         return;
     }
     if (n > SEG) {

@@ -591,11 +591,11 @@ __global__ __launch_bounds__(256) void k_modifier(u8 *obj, const u64 *begin, con
         const u32 sz = size[i];
         if (m.kind <= QD_MOD_ZGATE) {
             if (m.bit >= sz || (m.kind == QD_MOD_CNOT && m.control_bit >= sz)) {
-                atomicOr(err, ERR_BIT);
+                raise_error(err, ERR_BIT);
                 continue;
             }
         } else if (!qcgd_valid(o, sz)) {
-            atomicOr(err, ERR_OBJECT);
+            raise_error(err, ERR_OBJECT);
             continue;
         }
         double2 mm = mag[i];

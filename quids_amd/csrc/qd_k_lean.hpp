@@ -168,7 +168,7 @@ __device__ inline u64 lean_parent(const u64 *cb, const u64 *ctab, u64 c) {
 template <int KIND>
 __global__ __launch_bounds__(1024) void k_lean_generate(Parents P, const PDesc *D, const u64 *cb, const u64 *ctab,
                                                         const u64 *tab, qd_rule rule, LeanPlan *lp, u64 *cnt1,
-                                                        Entry *E1) {
+                                                        Entry *E1, u32 *slotof, u64 *off) {
     if (lean_stopped(lp, LEAN_GENERATE)) return;
     __shared__ u32 bcnt[256];
     __shared__ u64 bidx[256];
@@ -186,6 +186,7 @@ __global__ __launch_bounds__(1024) void k_lean_generate(Parents P, const PDesc *
         cplx m{0.0, 0.0};
         u32 d = 0, r = 0;
         if (c < C) {
+            if (slotof) slotof[c] = ~0u;
             const u64 p = lean_parent(cb, ctab, c);
             const u32 j = u32(c - cb[p]);
             const double2 m0 = P.mag[p];
@@ -221,6 +222,20 @@ __global__ __launch_bounds__(1024) void k_lean_generate(Parents P, const PDesc *
         __syncthreads();  // bcnt is cleared for the next chunk
     }
     if (spill) atomicOr(&lp->stop[LEAN_GENERATE], LEAN_SPILL);
+    // one pass: the last block to end turns the buckets' counts into offsets
+    // (a launch of its own cost 5 us).  The counts are read where the atomics
+    // leave them; each block's have returned before it takes its ticket.
+    if (!off) return;
+    __shared__ u64 tmp[1024 / kWave + 1];
+    if (threadIdx.x == 0) bcnt[0] = atomicAdd(&lp->ticket[2], 1u);
+    __syncthreads();
+    if (bcnt[0] != gridDim.x - 1) return;
+    const u32 nb = 1u << b1;
+    const u64 v = threadIdx.x < nb ? __hip_atomic_load(cnt1 + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    u64 total;
+    const u64 run = block_excl_scan(v, tmp, total);
+    if (threadIdx.x < nb) off[threadIdx.x] = run;
+    if (threadIdx.x == 0) off[nb] = total;
 }
 
 // Bucket offsets (exclusive prefix of the buckets' counts): one block.
@@ -469,10 +484,13 @@ __global__ __launch_bounds__(1024) void k_sel_finish(const SelItem *S, u32 ns, u
 // them, and two look-backs give its first rank and byte.  In place of a
 // bitmap, its popcount scan, the placement, the child sizes and the scan of
 // the sizes (eight launches): 24 us in place of 75 in a 12-node split_merge
-// step of 1.4e6 candidates and 2e4 survivors.
+// step of 1.4e6 candidates and 2e4 survivors.  Bound by a tile's chain of
+// dependent reads (ticket, slots, parent search, size, look-backs), so a tile
+// has 1024 threads: where every candidate survives, 256 of them took it in 16
+// rounds (2^17 hadamard children 21 us, now 13).
 // ---------------------------------------------------------------------------
 constexpr u32 kEmitTile = 4096;
-constexpr u32 kEmitThreads = 256;
+constexpr u32 kEmitThreads = 1024;
 
 template <int KIND>
 __global__ __launch_bounds__(kEmitThreads) void k_lean_emit(Parents P, const u64 *cb, const u64 *ctab,

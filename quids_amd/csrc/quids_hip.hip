@@ -321,6 +321,8 @@ static __device__ __align__(256) double scratch[kNoAllocDoubles];
 constexpr u64 kHostN = 8191;  // slot of the pinned area that stages a value for the device
 constexpr u64 kHostScan = 7960;  // reports of the device-driven step: the scan's, the last kernel's
 constexpr u64 kHostLean = 7968;
+constexpr u64 kHostSum = 7980;  // a canonical sum
+constexpr u64 kHostErr = 7981;  // a modifier's error word
 constexpr u64 kHostSegLoop = 8000;  // first of the slots that stage the batched select loop's state
 constexpr u64 kHostSelLoop = 8064;  // first of the slots that stage the select loop's state
 
@@ -563,20 +565,24 @@ static int canonical_sum(qd_ctx *ctx, const double2 *mag, const double *vals, u6
         QD_TRY(ctx->chunks.ensure(2 * cap * sizeof(double)));
         buf = ctx->chunks.as<double>();
     }
-    double *a = buf, *b = a + cap;
+    // the last level's sum goes to pinned memory, not waited for twice
+    double *a = buf, *b = a + cap, *const host = reinterpret_cast<double *>(ctx->host + kHostSum);
     prof_begin(ctx, QD_PHASE_NORMALIZE);
-    hipLaunchKernelGGL(k_sum_chunks, dim3(nchunk), dim3(kSumThreads), 0, ctx->stream, mag, vals, n, a);
+    hipLaunchKernelGGL(k_sum_chunks, dim3(nchunk), dim3(kSumThreads), 0, ctx->stream, mag, vals, n,
+                       nchunk == 1 ? host : a);
     u64 m = nchunk;
     while (m > 1) {
         const u64 nc2 = (m + kSumChunk - 1) / kSumChunk;
         hipLaunchKernelGGL(k_sum_chunks, dim3(nc2), dim3(kSumThreads), 0, ctx->stream, (const double2 *)nullptr,
-                           (const double *)a, m, b);
+                           (const double *)a, m, nc2 == 1 ? host : b);
         std::swap(a, b);
         m = nc2;
     }
     QD_HIP(hipGetLastError());
     prof_end(ctx, QD_PHASE_NORMALIZE);
-    QD_TRY(sync_read(ctx, a, sizeof(double), result));
+    QD_HIP(hipStreamSynchronize(ctx->stream));
+    prof_collect(ctx);
+    *result = *host;
     return QD_OK;
 }
 
@@ -923,7 +929,7 @@ static int dedup_phase(qd_ctx *ctx, const Entry *D, u64 rstride, const u64 *woff
     auto run_dedup = [&](auto kern, int threads) -> int {
         hipLaunchKernelGGL(kern, dim3(resident(kern, threads, nbk)), dim3(threads), 0, s, D, rstride, woff, nbk, L,
                            tol, UH, UR, UM, UK, counters, ctx->nhist.as<u64>(), ctx->biglist.as<u64>(),
-                           ctx->redolist.as<u64>(), (LeanPlan *)nullptr, (const Entry *)nullptr);
+                           ctx->redolist.as<u64>(), (LeanPlan *)nullptr, (const Entry *)nullptr, (u32 *)nullptr);
         QD_HIP(hipGetLastError());
         return QD_OK;
     };
@@ -2298,7 +2304,13 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
     u64 *UH = ctx->ebuf0.as<u64>();  // (the kernels place UR and UM after C of them)
     Entry *E1 = ctx->ebuf1.as<Entry>(), *E2 = two ? ctx->ebuf2.as<Entry>() : E1;
     u32 *UK = keys ? ctx->ukey.as<u32>() : nullptr;
-    u32 *slotof = ctx->ebuf1.as<u32>();  // (after the dedup has read its entries)
+    // by work items, or one child per lane
+    const bool items = KIND != QD_RULE_HADAMARD && C > kLeanChildMax;
+    // every unique survives: the dedup itself fills the map from candidates
+    // to slots, which the generate clears (else it takes the entries' place
+    // once the dedup has read them)
+    const bool all = !keys && !items;
+    u32 *slotof = all ? ctx->ukey.as<u32>() : ctx->ebuf1.as<u32>();
     u64 *nhist = a + la.nhist, *hist2 = a + la.hist2, *cnt1 = a + la.cnt1;
     if (C) {  // a fresh state: pooled buffers of about the size that a truncated step's survivors need
         out->begin.grow_from_pool((bound + 1) * sizeof(u64));
@@ -2311,7 +2323,7 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
     LeanReport *rep = reinterpret_cast<LeanReport *>(ctx->host + kHostLean);
 
     prof_begin(ctx, QD_PHASE_GENERATE);
-    if (KIND != QD_RULE_HADAMARD && C > kLeanChildMax) {
+    if (items) {
         const u64 nchunk = (nitems + kGenThreads - 1) / kGenThreads;
         QD_TRY(ensure_relieved(ctx, ctx->cpar, nchunk * sizeof(u64)));
         hipLaunchKernelGGL(k_chunk_parent, dim3(grid_for(nchunk)), dim3(256), 0, s, ctx->wb.as<u64>(), P.n, nchunk,
@@ -2325,7 +2337,7 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
     } else {
         hipLaunchKernelGGL(k_lean_generate<KIND>, dim3(grid_for(room, kLeanChunk, 1024)), dim3(kLeanChunk), 0, s, P,
                            (const PDesc *)ctx->pdesc.as<PDesc>(), cb, ctab, (const u64 *)ctx->tab.as<u64>(), rule, lp,
-                           cnt1, E1);
+                           cnt1, E1, all ? slotof : nullptr, two ? nullptr : ctx->off2.as<u64>());
     }
     QD_HIP(hipGetLastError());
     prof_end(ctx, QD_PHASE_GENERATE);
@@ -2334,23 +2346,26 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
         hipLaunchKernelGGL(k_level2_runs<kSplitBits>, dim3(kL2Grid), dim3(1024), 0, s, (const Entry *)E1, u64(0),
                            (const u64 *)cnt1, u64(0), 0u, 0u, u64(0), E2, cnt2, (u32 *)nullptr, (Entry *)nullptr,
                            (u64 *)nullptr, 1u, lp);
-    hipLaunchKernelGGL(k_lean_bscan, dim3(1), dim3(1024), 0, s, (const u64 *)cnt1, (const u64 *)cnt2,
-                       (const LeanPlan *)lp, ctx->off2.as<u64>());
+    if (two || items)  // (else the generate's last block has done it)
+        hipLaunchKernelGGL(k_lean_bscan, dim3(1), dim3(1024), 0, s, (const u64 *)cnt1, (const u64 *)cnt2,
+                           (const LeanPlan *)lp, ctx->off2.as<u64>());
     QD_HIP(hipGetLastError());
     prof_end(ctx, QD_PHASE_PARTITION);
     prof_begin(ctx, QD_PHASE_DEDUP);
     hipLaunchKernelGGL((k_dedup<512, 1024, 2048>), dim3(512), dim3(512), 0, s, (const Entry *)E1, u64(0),
                        (const u64 *)ctx->off2.as<u64>(), u64(0), 0u, prm.tolerance, UH, (u64 *)nullptr,
                        (double2 *)nullptr, UK, (u64 *)nullptr, nhist, ctx->biglist.as<u64>(), ctx->redolist.as<u64>(),
-                       lp, (const Entry *)E2);
+                       lp, (const Entry *)E2, all ? slotof : nullptr);
     QD_HIP(hipGetLastError());
     prof_end(ctx, QD_PHASE_DEDUP);
     prof_begin(ctx, QD_PHASE_SELECT);
     const unsigned gs = grid_for(room, 1024, 1024);
-    hipLaunchKernelGGL(k_lean_hist2, dim3(gs), dim3(256), 0, s, lp, (const u64 *)nhist, (const u32 *)UK, max_obj, hist2,
-                       slotof);
-    hipLaunchKernelGGL(k_lean_first, dim3(gs), dim3(256), 0, s, lp, (const u64 *)hist2, (const u32 *)UK,
-                       (const u64 *)UH, max_obj, ctx->sel0.as<SelItem>(), slotof);
+    if (!all) {
+        hipLaunchKernelGGL(k_lean_hist2, dim3(gs), dim3(256), 0, s, lp, (const u64 *)nhist, (const u32 *)UK, max_obj,
+                           hist2, slotof);
+        hipLaunchKernelGGL(k_lean_first, dim3(gs), dim3(256), 0, s, lp, (const u64 *)hist2, (const u32 *)UK,
+                           (const u64 *)UH, max_obj, ctx->sel0.as<SelItem>(), slotof);
+    }
     if (keys)
         hipLaunchKernelGGL(k_lean_finish, dim3(1), dim3(1024), 0, s, lp, (const SelItem *)ctx->sel0.as<SelItem>(),
                            max_obj, (const u64 *)UH, slotof);
@@ -3849,14 +3864,20 @@ int qd_ctx_set_phase_hook(qd_ctx *c, qd_phase_hook hook, void *user) {
     return QD_OK;
 }
 
+// A modifier's error word, in pinned memory: cleared and read by the host
+// itself, where a fill and a copy around a 2 us kernel took 13 of 27 us.
+static u32 *modifier_error(qd_ctx *c) {
+    u32 *w = reinterpret_cast<u32 *>(c->host + kHostErr);
+    *w = 0;
+    return w;
+}
+
 int qd_apply_modifier(qd_ctx *c, qd_state *s, const qd_modifier *m) {
     if (!c || !s || !m) return fail(QD_ERR_INVALID, "null argument");
     if (!modifier_known(m->kind)) return fail(QD_ERR_UNSUPPORTED, "modifier kind has no device implementation");
     QD_HIP(hipSetDevice(c->device));
     if (s->n == 0) return QD_OK;
-    QD_TRY(c->counters.ensure(64 * sizeof(u64)));
-    u32 *errw = reinterpret_cast<u32 *>(c->counters.as<u64>() + 4);
-    QD_HIP(hipMemsetAsync(errw, 0, sizeof(u32), c->stream));
+    u32 *errw = modifier_error(c);
     if (m->kind == QD_MOD_QCGD_STEP || m->kind == QD_MOD_QCGD_REVERSED_STEP)
         hipLaunchKernelGGL(k_step_modifier, dim3(grid_for(s->n, 16, 65536)), dim3(256), 0, c->stream,
                            s->objects.as<u8>(), s->begin.as<u64>(), s->size.as<u32>(), s->n, *m, errw);
@@ -3864,9 +3885,8 @@ int qd_apply_modifier(qd_ctx *c, qd_state *s, const qd_modifier *m) {
         hipLaunchKernelGGL(k_modifier, dim3(grid_for(s->n)), dim3(256), 0, c->stream, s->objects.as<u8>(),
                            s->begin.as<u64>(), s->size.as<u32>(), s->mag.as<double2>(), s->n, *m, errw);
     QD_HIP(hipGetLastError());
-    u32 w = 0;
-    QD_TRY(sync_read(c, errw, sizeof(u32), &w));
-    return check_err_word(w);
+    QD_HIP(hipStreamSynchronize(c->stream));
+    return check_err_word(*errw);
 }
 
 int qd_normalize(qd_ctx *c, qd_state *s, double *total_proba) {
@@ -3949,16 +3969,13 @@ int qd_modifier_adjoint(qd_ctx *c, qd_state *after, const qd_modifier *m, double
     if (after->n == 0) return QD_OK;
     if (!cot) return fail(QD_ERR_INVALID, "null cotangent");
     QD_HIP(hipSetDevice(c->device));
-    QD_TRY(c->counters.ensure(64 * sizeof(u64)));
-    u32 *errw = reinterpret_cast<u32 *>(c->counters.as<u64>() + 4);
-    QD_HIP(hipMemsetAsync(errw, 0, sizeof(u32), c->stream));
+    u32 *errw = modifier_error(c);
     hipLaunchKernelGGL(k_modifier_adjoint, dim3(grid_for(after->n)), dim3(256), 0, c->stream,
                        after->objects.as<u8>(), after->begin.as<u64>(), after->size.as<u32>(), after->n, *m,
                        reinterpret_cast<double2 *>(cot), errw);
     QD_HIP(hipGetLastError());
-    u32 w = 0;
-    QD_TRY(sync_read(c, errw, sizeof(u32), &w));
-    return check_err_word(w);
+    QD_HIP(hipStreamSynchronize(c->stream));
+    return check_err_word(*errw);
 }
 
 int qd_average_value(qd_ctx *c, qd_state *s, int observable, int arg, double *value, double *cot) {
