@@ -352,10 +352,11 @@ __device__ __attribute__((always_inline)) inline void group_reduce(u32 i, u32 j,
 //    registers, sorted by candidate index and summed pairwise in that order
 //    (the reference's canonical order);
 //  * members of larger groups append (slot << 52 | candidate << 12 | entry)
-//    to a wide area, sorted by (group, candidate) with a bitonic sort (in
-//    registers of one wavefront when it holds at most 64 entries, else
-//    block-wide in LDS) and summed by a segmented pairwise tree in that
-//    order.
+//    to a wide area, sorted by (group, candidate) and summed by a segmented
+//    pairwise tree in that order.  Up to 64 entries are ranked and summed by
+//    one wavefront, up to T / 2 ranked by all (each entry counts the smaller
+//    ones); a bitonic sort in LDS, 28 barriers at 128 entries, is left to
+//    more.
 // Groups with |m|^2 > tol (hash, smallest candidate index, sum) go to the
 // front of the bucket's output range (one LDS counter), the rest of the
 // range gets the sentinel representative ~0.  A bucket whose candidate
@@ -363,6 +364,12 @@ __device__ __attribute__((always_inline)) inline void group_reduce(u32 i, u32 j,
 // (counted in counters[6]) for k_dedup_sort and writes nothing; one beyond
 // the LDS capacity goes to biglist (counters[5]).  Layout of E, woff and
 // the output as in k_dedup_sort.
+//
+// Bound by its chain of barriers and LDS accesses per bucket (two workgroups
+// of 8 wavefronts a CU, 70 % of their cycles waiting).  3.3e8 split_merge
+// candidates in 1.5e8 groups 11.5 ms (13.5 with a bitonic sort of every wide
+// area), 2.7e8 erase_create candidates in 2.5e8 groups 5.2 ms (16.5 GB read
+// and written).
 constexpr int kWideCandBits = 40;
 
 template <int T, int CAP, int TS>
@@ -526,14 +533,11 @@ __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const 
                 const u32 l = threadIdx.x;
                 const bool valid = l < W;
                 u64 v = valid ? wkey[l] : ~0ull;
-#pragma unroll
-                for (u32 kk = 2; kk <= u32(kWave); kk <<= 1) {
-#pragma unroll
-                    for (u32 jj = kk >> 1; jj > 0; jj >>= 1) {
-                        const u64 o = __shfl_xor(v, int(jj), kWave);
-                        v = (((l & jj) == 0) == ((l & kk) == 0)) ? min(v, o) : max(v, o);
-                    }
-                }
+                u32 rank = 0;
+                for (u32 j = 0; j < W; ++j) rank += wkey[j] < v;
+                if (valid) wkey[rank] = v;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                v = valid ? wkey[l] : ~0ull;
                 const u32 sl = u32(v >> 52);
                 const u32 psl = __shfl_up(sl, 1, kWave);
                 u32 g0 = (l == 0 || psl != sl) ? l : 0u;  // group start lane: running max of the starts
@@ -561,22 +565,41 @@ __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const 
             }
             __syncthreads();
         } else if (W) {
-            u32 P = 1;
-            while (P < W) P <<= 1;
-            for (u32 q = W + threadIdx.x; q < P; q += T) wkey[q] = ~0ull;
-            __syncthreads();
-            for (u32 kk = 2; kk <= P; kk <<= 1) {
-                for (u32 jj = kk >> 1; jj > 0; jj >>= 1) {
-                    for (u32 t = threadIdx.x; t < P / 2; t += T) {
-                        const u32 lo = ((t & ~(jj - 1)) << 1) | (t & (jj - 1));
-                        const u32 hi = lo | jj;
-                        const u64 va = wkey[lo], vb = wkey[hi];
-                        if ((va > vb) == ((lo & kk) == 0)) {
-                            wkey[lo] = vb;
-                            wkey[hi] = va;
+            if (W <= u32(T) / 2) {
+                // every entry counts the smaller ones, T / pitch threads each
+                // (a bitonic sort of 128 entries takes 28 barriers)
+                const u32 pitch = (W + kWave - 1) / kWave * kWave, np = T / pitch;
+                const u32 q = threadIdx.x % pitch, part = threadIdx.x / pitch;
+                if (threadIdx.x < W) lnk[threadIdx.x] = 0;
+                __syncthreads();
+                u64 v = 0;
+                if (q < W && part < np) {
+                    v = wkey[q];
+                    u32 rank = 0;
+                    for (u32 j = part * W / np; j < (part + 1) * W / np; ++j) rank += wkey[j] < v;
+                    if (rank) atomicAdd(&lnk[q], rank);
+                }
+                __syncthreads();
+                if (threadIdx.x < W) wkey[lnk[threadIdx.x]] = v;
+                __syncthreads();
+            } else {
+                u32 P = 1;
+                while (P < W) P <<= 1;
+                for (u32 q = W + threadIdx.x; q < P; q += T) wkey[q] = ~0ull;
+                __syncthreads();
+                for (u32 kk = 2; kk <= P; kk <<= 1) {
+                    for (u32 jj = kk >> 1; jj > 0; jj >>= 1) {
+                        for (u32 t = threadIdx.x; t < P / 2; t += T) {
+                            const u32 lo = ((t & ~(jj - 1)) << 1) | (t & (jj - 1));
+                            const u32 hi = lo | jj;
+                            const u64 va = wkey[lo], vb = wkey[hi];
+                            if ((va > vb) == ((lo & kk) == 0)) {
+                                wkey[lo] = vb;
+                                wkey[hi] = va;
+                            }
                         }
+                        __syncthreads();
                     }
-                    __syncthreads();
                 }
             }
             // group starts in the sorted area (the owner slots are free now)

@@ -1,13 +1,16 @@
-"""The second radix pass over its range of sub-bucket counts: up to 2^10 (two
+"""The partition and dedup over their ranges.  The second radix pass over its range of sub-bucket counts: up to 2^10 (two
 workgroups a CU), 2^11 (one), beyond (entries written directly), and several
 workgroups to a bucket in the hash-range passes, all the same final state as
 the default layout."""
 import math
 
+import numpy as np
 import pytest
 
 import quids_amd as q
+from oracle import oracle as orc
 from quids_amd.rules import qcgd
+from quids_amd.rules import quantum_computer as qc
 from quids_amd.state import HostState
 
 from helpers import assert_states_identical
@@ -57,3 +60,34 @@ def test_sub_bucket_counts(parents, first_pass_bits):
 def test_range_groups(parents, chunk_log2):
     got = _final(parents, dedup_bucket_target=64, chunk_log2=chunk_log2)
     assert_states_identical(got, _final(parents), f"passes of 2^{chunk_log2}")
+
+
+# groups beyond the registers' eight members, in the LDS table of each size:
+# ranked by one wavefront (up to 64 entries), by all threads (up to half of
+# them), sorted beyond
+@pytest.mark.parametrize("dedup_cap", [256, 512, 1024, 2048])
+@pytest.mark.parametrize("copies", [9, 31, 32, 33, 63, 64, 65, 127, 128, 129, 240])
+def test_groups_of_equal_hashes(copies, dedup_cap):
+    rng = np.random.default_rng(copies)
+    n = 4 * copies
+    reg = np.zeros((n, 8), np.uint8)
+    # a few registers share each hash: `copies` of one, and groups of 1 to 12
+    kinds = np.concatenate([np.zeros(copies), 1 + rng.integers(0, n // 4, n - copies)]).astype(np.uint32)
+    kinds = rng.permutation(kinds)
+    reg[:, 1], reg[:, 2] = kinds & 0xFF, kinds >> 8
+    reg[:, 0] = rng.integers(0, 2, n)
+    mag = rng.normal(size=n) + 1j * rng.normal(size=n)
+    hs = HostState(reg.reshape(-1), np.arange(n + 1, dtype=np.uint64) * np.uint64(8), np.full(n, 4, np.uint32),
+                   mag / np.linalg.norm(mag))
+    ctx = q.default_context()
+    old = ctx.get_tuning()
+    ctx.set_tuning(dedup_bucket_target=min(dedup_cap // 2, 512), dedup_cap=dedup_cap)
+    try:
+        a, b = q.it_t(), q.it_t()
+        a.upload(hs)
+        st = q.simulate(a, qc.hadamard(0), b)
+        ref, ost = orc.simulate(hs, qc.hadamard(0))
+        assert st["num_unique"] == ost["num_unique"]
+        assert_states_identical(b.download(), ref, f"{copies} copies, table of {dedup_cap}")
+    finally:
+        ctx.set_tuning(dedup_bucket_target=old["dedup_bucket_target"], dedup_cap=old["dedup_cap"])
