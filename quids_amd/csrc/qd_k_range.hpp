@@ -14,60 +14,90 @@
 
 namespace qd {
 
-constexpr int kPoolPer = 16;  // slots per thread of k_pool_append
+constexpr u32 kPoolThreads = 512;
+constexpr u32 kPoolGrid = 512;  // blocks, at most
 
 // Appends the slots holding a unique (UR != kNoRep) to the pool: hash (the
 // slot key rotated back), representative, magnitude and, with UK, the top
-// 32 |m|^2 bits, in slot order within a block tile of 256 * kPoolPer slots,
-// so that the uniques of one wavefront's 64 slots land side by side
-// (coalesced stores).  One reservation per tile.  With UK, a unique whose
-// top 24 |m|^2 bits are below t24 is left out: the pool already holds
-// max_num_object keys at or above that prefix, so it can never be kept.
-__global__ __launch_bounds__(256) void k_pool_append(const u64 *SK, const u64 *UR, const double2 *UM, const u32 *UK,
-                                                     u32 t24, u64 nslots, u64 *Ph, u64 *Pr, double2 *Pm, u32 *Pk,
-                                                     u64 *pcount) {
-    constexpr int kWaves = 256 / kWave;
-    constexpr int kRuns = kPoolPer * kWaves;  // runs of 64 slots in a tile, in slot order
-    static_assert(kRuns == kWave, "one lane of the first wavefront per run");
-    __shared__ u64 roff[kRuns];  // count, then exclusive prefix, of each run's uniques
+// 32 |m|^2 bits, in slot order within a wavefront's run of slots (coalesced
+// stores).  With UK, a unique whose top 24 |m|^2 bits are below t24 is left
+// out: the pool already holds max_num_object keys at or above that prefix, so
+// it can never be kept.  A block counts its run's first and reserves its
+// places with one addition: one for every 4096 slots, to the same word, took
+// 45 us of a group of 7.3e6 slots of which few are kept.
+__global__ __launch_bounds__(kPoolThreads) void k_pool_append(const u64 *SK, const u64 *UR, const double2 *UM,
+                                                              const u32 *UK, u32 t24, u64 nslots, u64 *Ph, u64 *Pr,
+                                                              double2 *Pm, u32 *Pk, u64 *pcount) {
+    constexpr u32 kWaves = kPoolThreads / kWave, kRows = 16;
+    __shared__ u64 wcnt[kWaves];
     __shared__ u64 base;
-    constexpr u64 kTile = 256 * kPoolPer;
     const u32 lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    const u64 below = (1ull << lane) - 1;
-    for (u64 t0 = u64(blockIdx.x) * kTile; t0 < nslots; t0 += u64(gridDim.x) * kTile) {
-        u64 r[kPoolPer], m[kPoolPer];
+    const u64 nwave = u64(gridDim.x) * kWaves, w = u64(blockIdx.x) * kWaves + wid;
+    const u64 per = (nslots + nwave * kWave - 1) / (nwave * kWave) * kWave;
+    const u64 i0 = min(w * per, nslots), i1 = min(i0 + per, nslots);
+    // which of a lane's kRows slots to keep (bit q: slot r + 64 q + lane), and
+    // their keys.  The 4-byte key first: below t24, the slot, empty or not, is
+    // left out without reading its representative; at or above t24 it is a
+    // unique.  (All loads of the rows are issued before any is looked at.)
+    auto rows = [&](u64 r, u32 (&key)[kRows]) {
+        u32 keep = 0;
+        u64 at[kRows];
 #pragma unroll
-        for (int k = 0; k < kPoolPer; ++k) {
-            const u64 i = t0 + threadIdx.x + 256 * k;
-            // (with UK, the 4-byte key first: below t24, the slot, empty or
-            // not, is left out without reading its representative)
-            r[k] = kNoRep;
-            if (i < nslots && (!UK || (UK[i] >> 8) >= t24)) r[k] = UR[i];
-            m[k] = __ballot(r[k] != kNoRep);
-            if (lane == 0) roff[k * kWaves + wid] = __popcll(m[k]);
-        }
-        __syncthreads();
-        if (wid == 0) {
-            const u64 c = roff[lane];
-            const u64 inc = wave_incl_scan(c);
-            roff[lane] = inc - c;
-            if (lane == kWave - 1)
-                base = inc ? atomicAdd(reinterpret_cast<unsigned long long *>(pcount), (unsigned long long)inc) : 0;
-        }
-        __syncthreads();
-        const u64 b = base;
+        for (u32 q = 0; q < kRows; ++q) at[q] = min(r + q * kWave + lane, i1 - 1);
+        if (UK) {
 #pragma unroll
-        for (int k = 0; k < kPoolPer; ++k) {
-            if (r[k] != kNoRep) {
-                const u64 i = t0 + threadIdx.x + 256 * k;
-                const u64 at = b + roff[k * kWaves + wid] + __popcll(m[k] & below);
+            for (u32 q = 0; q < kRows; ++q) key[q] = UK[at[q]];
+        }
+        if (UK && t24) {
+#pragma unroll
+            for (u32 q = 0; q < kRows; ++q) keep |= u32(key[q] >> 8 >= t24) << q;
+        } else {
+            u64 rep[kRows];
+#pragma unroll
+            for (u32 q = 0; q < kRows; ++q) rep[q] = UR[at[q]];
+#pragma unroll
+            for (u32 q = 0; q < kRows; ++q) keep |= u32(rep[q] != kNoRep) << q;
+        }
+#pragma unroll
+        for (u32 q = 0; q < kRows; ++q)
+            if (r + q * kWave + lane >= i1) keep &= ~(1u << q);
+        return keep;
+    };
+    u64 cnt = 0;
+    u32 key[kRows];
+    for (u64 r = i0; r < i1; r += kRows * kWave) cnt += u32(__popc(rows(r, key)));
+#pragma unroll
+    for (int o = kWave / 2; o; o >>= 1) cnt += __shfl_xor(cnt, o, kWave);
+    if (lane == 0) wcnt[wid] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        u64 sum = 0;
+        for (u32 q = 0; q < kWaves; ++q) {
+            const u64 v = wcnt[q];
+            wcnt[q] = sum;
+            sum += v;
+        }
+        base = sum ? atomicAdd(reinterpret_cast<unsigned long long *>(pcount), (unsigned long long)sum) : 0;
+    }
+    __syncthreads();
+    if (!cnt) return;
+    u64 at0 = base + wcnt[wid];
+    for (u64 r = i0; r < i1; r += kRows * kWave) {
+        const u32 keep = rows(r, key);
+        if (__ballot(keep != 0) == 0) continue;
+#pragma unroll
+        for (u32 q = 0; q < kRows; ++q) {
+            const bool kept = (keep >> q) & 1u;
+            const u64 m = __ballot(kept);
+            if (kept) {
+                const u64 i = r + q * kWave + lane, at = at0 + __popcll(m & ((1ull << lane) - 1));
                 Ph[at] = rotr12(SK[i]);
-                Pr[at] = r[k];
+                Pr[at] = UR[i];
                 Pm[at] = UM[i];
-                if (UK) Pk[at] = UK[i];
+                if (UK) Pk[at] = key[q];
             }
+            at0 += __popcll(m);
         }
-        __syncthreads();  // roff and base are rewritten by the next tile
     }
 }
 

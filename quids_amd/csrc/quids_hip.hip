@@ -1432,7 +1432,8 @@ __global__ __launch_bounds__(256) void k_add_offset(const u64 *src, u64 n, u64 a
 // sub-buckets' slack and of the group's 32-bit select keys and pool
 // appends.
 constexpr u32 kRangeGroups = 8;
-constexpr double kRangeBytesPerCand = 32.0 * 1.03 + (32.0 + 32.0 * 2.05 + 4.0 + 36.0) / kRangeGroups;
+constexpr double range_bytes_per_cand(u32 groups) { return 32.0 * 1.03 + (32.0 + 32.0 * 2.05 + 4.0 + 36.0) / groups; }
+constexpr double kRangeBytesPerCand = range_bytes_per_cand(kRangeGroups);
 
 template <int KIND>
 static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule &rule, u64 C, u64 nitems,
@@ -1492,11 +1493,15 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
     if (fill_tab) slabbed.push_back(&ctx->tab);
     u64 slab_want = ctx->slab.cap;
     double log_free = 0, log_reuse = 0, log_fixed = 0;  // the plan's inputs, for QD_LOG_RANGE
+    u32 groups = kRangeGroups;  // of a pass
     if (ctx->tune.chunk_log2) {
         budget = 1ull << ctx->tune.chunk_log2;
         T = tag_bits(budget);
+        // (passes this small leave memory: groups of about 8e6 candidates,
+        // whose waits and small launches weigh less than in more groups)
+        while (groups > 1 && budget / groups < (1u << 22) + (1u << 21)) groups /= 2;
         const double need = double(tab_bytes) + double(T) * double(pstride) + pool_bytes +
-                            kSlabSlack * kRangeBytesPerCand * double(budget) + double(64ull << 20);
+                            kSlabSlack * range_bytes_per_cand(groups) * double(budget) + double(64ull << 20);
         slab_want = std::max<u64>(slab_want, u64(need));
     } else {
         ctx->pool.trim();
@@ -1660,7 +1665,7 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
     // the two-walk way's first-level buckets: all in the regions' memory
     const u32 nparts = 1, pshift = b1;
     const u64 perpart = nb1;
-    const u32 ngroups = u32(std::min<u64>(nb1, kRangeGroups));
+    const u32 ngroups = u32(std::min<u64>(nb1, groups));
     const u64 gbk = nb1 / ngroups;  // first-level buckets per group (a group lies in one part)
     const double gmean = double(nmax) / double(ngroups);
     const u64 gcap = u64(gmean * 1.02 + 8.0 * std::sqrt(gmean)) + 4096;  // entries of a group, at most
@@ -1939,9 +1944,8 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
             ns = hb[8];  // the pool as the groups before this one left it
             if (!U) continue;
             if (capped && (ns > 2 * max_obj || ns + ng > pcap)) QD_TRY(trim_pool());
-            hipLaunchKernelGGL(k_pool_append,
-                               dim3(unsigned(std::min<u64>((ng + 256 * kPoolPer - 1) / (256 * kPoolPer), 16384))),
-                               dim3(256), 0, s, (const u64 *)UH, (const u64 *)UR, (const double2 *)UM, (const u32 *)UK,
+            hipLaunchKernelGGL(k_pool_append, dim3(grid_for(ng, kPoolThreads * 8, kPoolGrid)), dim3(kPoolThreads), 0, s,
+                               (const u64 *)UH, (const u64 *)UR, (const double2 *)UM, (const u32 *)UK,
                                t24, ng, Ph, Pr, Pm, Pk, pcount);
             QD_HIP(hipGetLastError());
         }

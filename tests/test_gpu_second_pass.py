@@ -62,6 +62,31 @@ def test_range_groups(parents, chunk_log2):
     assert_states_identical(got, _final(parents), f"passes of 2^{chunk_log2}")
 
 
+# passes of several groups, whose pool is trimmed (a few of a group's uniques
+# are above its bound)
+@pytest.mark.parametrize("cap,chunk_log2", [(150000, 22), (300000, 24)])
+def test_range_pool(parents, cap, chunk_log2):
+    ctx = q.default_context()
+    old = ctx.get_tuning()
+    a, rule = q.it_t(), qcgd.erase_create(0.9, 0.4)
+    q.simulate(parents[0], parents[1], a, None, cap)
+    q.simulate(a, qcgd.step)
+    out = {}
+    try:
+        for log2 in (0, chunk_log2):
+            ctx.set_tuning(chunk_log2=log2)
+            b = q.it_t()
+            st = q.simulate(a, rule, b, None, cap)
+            out[log2] = b.download()
+            b.close()
+            if log2:
+                assert st["reserved"] & 4 and st["num_candidates"] > 2 << log2
+    finally:
+        ctx.set_tuning(chunk_log2=old["chunk_log2"])
+        a.close()
+    assert_states_identical(out[chunk_log2], out[0], f"cap {cap}")
+
+
 # groups beyond the registers' eight members, in the LDS table of each size:
 # ranked by one wavefront (up to 64 entries), by all threads (up to half of
 # them), sorted beyond
