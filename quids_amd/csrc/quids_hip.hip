@@ -2536,6 +2536,12 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     // (what the caller lets one pass take; hadamard steps have one pass only)
     const u64 lean_max = fast && ctx->tune.chunk_log2 ? std::min<u64>(kLeanMax, 1ull << ctx->tune.chunk_log2) : kLeanMax;
     if (room > lean_max) room = 0;
+    // (a device-driven step keeps to buffers of its own: views into the slab
+    // of the hash-range passes go when an allocation does not fit beside it,
+    // or the step falls back)
+    if (lean)
+        for (DBuf *b : {&ctx->ebuf2, &ctx->ukey})
+            if (b->view) b->release();
     const LeanArea la(N);
     QD_TRY(ensure_relieved(ctx, ctx->lean, la.words * sizeof(u64)));
     QD_TRY(ensure_relieved(ctx, ctx->ctab, kLeanTab * sizeof(u64)));

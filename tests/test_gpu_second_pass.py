@@ -116,3 +116,41 @@ def test_groups_of_equal_hashes(copies, dedup_cap):
         assert_states_identical(b.download(), ref, f"{copies} copies, table of {dedup_cap}")
     finally:
         ctx.set_tuning(dedup_bucket_target=old["dedup_bucket_target"], dedup_cap=old["dedup_cap"])
+
+
+def test_small_steps_after_hash_range_passes(parents):
+    """A hash-range step leaves its buffers with the context; the steps after
+    it, among them one whose select the device hands back (more equal keys
+    than one block takes), are the same as without them."""
+    ctx = q.default_context()
+    old = ctx.get_tuning()
+
+    def chain():
+        cur = q.it_t()
+        cur.upload(HostState.from_objects([qcgd.seeded_graph(10, 42)]))
+        for k in range(4):
+            if k % 2 == 0:
+                q.simulate(cur, qcgd.step)
+            nxt = q.it_t()
+            q.simulate(cur, [qcgd.split_merge(math.pi / 4, 0.0), qcgd.erase_create(math.pi / 3, math.pi / 5)][k % 2],
+                       nxt, None, 1 << 18)
+            cur.close()
+            cur = nxt
+        out = cur.download()
+        cur.close()
+        return out
+
+    ref = chain()
+    a = q.it_t()
+    q.simulate(parents[0], parents[1], a, None, 150000)
+    ctx.set_tuning(chunk_log2=22)
+    try:
+        b = q.it_t()
+        st = q.simulate(a, qcgd.erase_create(0.9, 0.4), b, None, 150000)
+        assert st["reserved"] & 4
+        for s in (a, b):
+            s.close()
+    finally:
+        ctx.set_tuning(chunk_log2=old["chunk_log2"])
+    for k in range(2):
+        assert_states_identical(chain(), ref, f"after a hash-range step, {k}")
