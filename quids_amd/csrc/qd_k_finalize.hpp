@@ -301,7 +301,8 @@ __global__ __launch_bounds__(kWave) void k_populate_flip(Parents P, const PDesc 
 // has nodes: 16, 32 or 64) writes one survivor at a time, lane i for the
 // parent's node i.
 constexpr u32 kPopNodes = 64;  // child nodes of a survivor in the lists
-constexpr u32 kPopSubs = 128;  // sub_nodes of its names
+constexpr u32 kPopSubs = 384;   // sub_nodes of its names (beyond, one lane writes the child: with 128, a batch of
+                                // 256 instances whose names had grown took 4.8 ms a step to write, now 0.5)
 
 // A name tree of the child: an optional new root over the parent's sub_nodes
 // [sb, sb + len) and [sb2, sb2 + len2).

@@ -114,7 +114,7 @@ def test_large_steps_match_the_host_driven_path(parents):
 
 # survivors' bytes: graphs around the lane segments' widths (16, 32, 64 nodes;
 # beyond, the whole step runs on the generic kernels), children beyond the
-# lists of 64 nodes and 128 names, at every alignment
+# lists of 64 nodes, at every alignment
 @pytest.mark.parametrize("align", [1, 2, 4, 8, 16])
 @pytest.mark.parametrize("nodes", [(1, 2), (15, 16), (16, 17), (31, 32, 33), (60, 63, 64), (64, 65)])
 def test_populate_widths(nodes, align):
@@ -169,3 +169,18 @@ def test_overflowing_sub_buckets(copies, exact, eager):
     assert st["num_unique"] == ost["num_unique"]
     assert bool(st["reserved"] & 1) == exact or st["reserved"] & 8
     assert_states_identical(g, o, f"copies {copies}")
+
+
+def test_populate_long_names():
+    """Children whose names grow from 36 sub_nodes past the lists' 384."""
+    hs = qcgd_initial(16, 42)
+    names = []
+    for k in range(80):
+        rule = qcgd.split_merge(1.56, 0.3) if k % 2 == 0 else qcgd.coin(0.3, 0.4)
+        ref = orc.simulate(hs, rule, 12)[0]
+        names.append(int(max(ref.object_size)) // 16)
+        if k % 2 == 0 and k % 4 == 0:
+            g, _ = _step(hs, rule, 12)
+            assert_states_identical(g, ref, f"step {k}, {names[-1]} names")
+        hs = orc.apply_modifier(ref, qcgd.step)
+    assert max(names) > 400
