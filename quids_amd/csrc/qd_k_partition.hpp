@@ -304,21 +304,12 @@ __global__ __launch_bounds__(kSplitThreads, 8) void k_region_place(const Entry *
 // lane writes its entries directly.  Arguments as k_level2_runs.
 __global__ __launch_bounds__(1024) void k_level2_fixed(const Entry *in, u64 in_stride, const u64 *off1, u64 nbk1,
                                                        u32 b1, u32 b2, u64 cap2, Entry *out, u64 *cnt2, u32 *err,
-                                                       Entry *ovf, u64 *ovf_n, LeanPlan *lp) {
-    if (lp) {  // a step driven from the device: off1 holds the buckets' counts
-        if (lean_stopped(lp, LEAN_LEVEL2) || lp->b2 == 0) return;
-        in_stride = lp->cap1;
-        b1 = lp->b1;
-        b2 = lp->b2;
-        cap2 = lp->cap2;
-        nbk1 = 1ull << b1;
-        err = &lp->stop[LEAN_LEVEL2];
-    }
+                                                       Entry *ovf, u64 *ovf_n) {
     __shared__ u32 ccnt[kLevel2Bins];
     __shared__ u32 cur[kLevel2Bins];
     bool spill = false;
     for (u64 b = blockIdx.x; b < nbk1; b += gridDim.x) {
-        const u64 beg = lp ? 0 : off1[b], end = lp ? off1[b] : off1[b + 1];
+        const u64 beg = off1[b], end = off1[b + 1];
         const u64 ibase = in_stride ? b * in_stride : beg;  // entry i of [beg, end) is in[ibase + i - beg]
         const u32 nb2 = 1u << b2;
         const u32 shift = 64 - b1 - b2;
@@ -414,7 +405,7 @@ __global__ __launch_bounds__(1024) void k_level2_fixed(const Entry *in, u64 in_s
         for (u32 i = threadIdx.x; i < nb2; i += blockDim.x) cnt2[(b << b2) + i] = ovf ? cur[i] : min<u64>(cur[i], cap2);
         __syncthreads();  // cur is cleared for the next bucket
     }
-    if (spill) atomicOr(err, lp ? LEAN_SPILL : ERR_SPILL);
+    if (spill) atomicOr(err, ERR_SPILL);
 }
 
 // The same split with exact offsets (a counting pass first): used when a

@@ -989,7 +989,7 @@ static int level2(qd_ctx *ctx, const Entry *in, u64 in_stride, const u64 *off1, 
     else
         hipLaunchKernelGGL(k_level2_fixed, dim3(unsigned(std::min<u64>(nbk1, 128))), dim3(1024), 0, ctx->stream, in,
                            in_stride, off1, nbk1, b1, b2, cap2, E2, ctx->cnt2.as<u64>(), errw, ctx->ovf.as<Entry>(),
-                           counters + 7, (LeanPlan *)nullptr);
+                           counters + 7);
     QD_HIP(hipGetLastError());
     return QD_OK;
 }
