@@ -4,6 +4,7 @@
 
 #include "qd_device.hpp"
 #include "qd_rules.hpp"
+#include "qd_sizes.hpp"
 
 namespace qd {
 
@@ -39,12 +40,6 @@ __global__ __launch_bounds__(256) void k_place(const u64 *UR, const double2 *UM,
             }
         }
     }
-}
-
-__device__ inline u32 align_pad(u32 size, u32 align) {
-    if (align <= 1) return 0;
-    const u32 off = align - size % align;
-    return off == align ? 0 : off;
 }
 
 template <int KIND>

@@ -502,8 +502,8 @@ __global__ __launch_bounds__(kEmitThreads) void k_lean_emit(Parents P, const u64
     constexpr u32 kPer = kEmitTile / kEmitThreads, kWaves = kEmitThreads / kWave, kRuns = kEmitTile / kWave;
     static_assert(kRuns == kWave, "one lane of the first wavefront per run of 64 candidates");
     // the tile's survivors, in order: dedup slot, candidate in the tile,
-    // parent beyond the tile's first, size, first byte in the tile
-    __shared__ u32 lslot[kEmitTile], lsize[kEmitTile], lpar[kEmitTile], lbyte[kEmitTile];
+    // parent beyond the tile's first, size
+    __shared__ u32 lslot[kEmitTile], lsize[kEmitTile], lpar[kEmitTile];
     __shared__ u16 loff[kEmitTile];
     __shared__ u32 roff[kRuns + 1];
     __shared__ u64 tmp[kWaves + 1], pre[2];
@@ -562,14 +562,9 @@ __global__ __launch_bounds__(kEmitThreads) void k_lean_emit(Parents P, const u64
         // byte offsets within the tile: each thread a run of the list
         const u32 per = (cnt + kEmitThreads - 1) / kEmitThreads;
         const u32 q0 = min(threadIdx.x * per, cnt), q1 = min(q0 + per, cnt);
-        u64 bytes = 0;
-        for (u32 q = q0; q < q1; ++q) bytes += lsize[q] + align_pad(lsize[q], align);
-        u64 total;
-        u64 run = block_excl_scan(bytes, tmp, total);
-        for (u32 q = q0; q < q1; ++q) {
-            lbyte[q] = u32(run);
-            run += lsize[q] + align_pad(lsize[q], align);
-        }
+        u64 at[kPer], total;
+        const u64 bytes = place_run(lsize + q0, q1 - q0, align, at);
+        const u64 run = block_excl_scan(bytes, tmp, total);
         if (wid == 0) {
             const u64 e = lookback<kWideVal>(dk, tile, cnt, 0);
             if (lane == 0) pre[0] = e;
@@ -585,9 +580,11 @@ __global__ __launch_bounds__(kEmitThreads) void k_lean_emit(Parents P, const u64
             orep[r] = c0 + loff[q];
             opar[r] = p0 + lpar[q];
             osize[r] = lsize[q];
-            obegin[r] = y0 + lbyte[q];
             omag[r] = UM[lslot[q]];
         }
+#pragma unroll
+        for (u32 k = 0; k < kPer; ++k)
+            if (q0 + k < q1 && r0 + q0 + k < capk) obegin[r0 + q0 + k] = y0 + run + at[k];
         if (tile == ntile - 1 && threadIdx.x == 0) {
             lp->K = r0 + cnt;
             lp->bytes = y0 + total;

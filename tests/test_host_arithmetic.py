@@ -1,0 +1,30 @@
+"""Plain integer arithmetic of the library (tests/cpp/host_checks.cpp), on the CPU."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+
+
+@pytest.fixture(scope="module")
+def lib():
+    so = os.path.join(CPP, "libhost_checks.so")
+    if not os.path.exists(so):
+        subprocess.run(["make", "-C", CPP, "libhost_checks.so"], check=True)
+    return ctypes.CDLL(so)
+
+
+# sums of sizes and padding at and beyond 2^32
+@pytest.mark.parametrize("align", [1, 8, 1 << 20])
+@pytest.mark.parametrize("size", [[], [5], [1, 2, 3, 4], [600 << 20] * 4, [2 ** 32 - 1] * 4, [2 ** 32 - 1, 1, 2 ** 31]])
+def test_places_of_objects(lib, size, align):
+    at = (ctypes.c_uint64 * 4)()
+    lib.host_place_run.restype = ctypes.c_uint64
+    end = lib.host_place_run((ctypes.c_uint32 * 4)(*size), len(size), align, at)
+    want = 0
+    for k, s in enumerate(size):
+        assert at[k] == want
+        want += (s + align - 1) // align * align
+    assert end == want
