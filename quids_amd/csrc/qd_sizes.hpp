@@ -31,4 +31,15 @@ QD_HD u64 place_run(const u32 *size, u32 n, u32 align, u64 (&at)[PER]) {
     return end;
 }
 
+// Objects that a state's begin, size and magnitude buffers of these bytes
+// hold (begin has one entry more than there are objects; a buffer whose
+// allocation failed has 0 bytes).
+QD_HD u64 state_room(u64 begin, u64 size, u64 mag) {
+    u64 n = begin / sizeof(u64);
+    if (n) --n;
+    if (size / sizeof(u32) < n) n = size / sizeof(u32);
+    if (mag / (2 * sizeof(double)) < n) n = mag / (2 * sizeof(double));
+    return n;
+}
+
 }  // namespace qd

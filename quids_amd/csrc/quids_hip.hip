@@ -2322,6 +2322,7 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
         out->mag.grow_from_pool(bound * sizeof(double2));
         out->objects.grow_from_pool(u64(1.2 * double(bound) * (double(in_bytes) / double(P.n) + 8)));
     }
+    QD_TRY(state_reserve(out, 0, 0));  // (the order writes obegin[0] at least; a failed growth leaves no buffer)
     u64 *cnt2 = two ? ctx->cnt2.as<u64>() : cnt1;
     const u64 *cb = ctx->cb.as<u64>(), *ctab = ctx->ctab.as<u64>();
     LeanReport *rep = reinterpret_cast<LeanReport *>(ctx->host + kHostLean);
@@ -2378,8 +2379,7 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
     for (int attempt = 0;; ++attempt) {
         // the output's room, as it is; when it is too small it grows to what
         // the survivors need, and these kernels run again
-        const u64 capk = std::min<u64>(std::min<u64>(out->begin.cap / sizeof(u64) - 1, out->size.cap / sizeof(u32)),
-                                       std::min<u64>(out->mag.cap / sizeof(double2), bound));
+        const u64 capk = std::min(state_room(out->begin.cap, out->size.cap, out->mag.cap), bound);
         const u64 capb = out->objects.cap;
         double *sums = ctx->chunks.as<double>();
         prof_begin(ctx, QD_PHASE_ORDER);

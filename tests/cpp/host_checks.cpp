@@ -8,3 +8,7 @@ extern "C" uint64_t host_place_run(const uint32_t *size, uint32_t n, uint32_t al
     for (int k = 0; k < 4; ++k) at[k] = a[k];
     return end;
 }
+
+extern "C" uint64_t host_state_room(uint64_t begin, uint64_t size, uint64_t mag) {
+    return qd::state_room(begin, size, mag);
+}

@@ -1,0 +1,62 @@
+"""Steps on a device whose memory is nearly taken by others: allocations that
+fail are errors or another way of running the step, and leave the states
+usable."""
+import contextlib
+
+import numpy as np
+import pytest
+import torch
+
+import quids_amd as q
+from oracle import oracle as orc
+from quids_amd._abi import QD_ERR_OOM, QuidsError
+from quids_amd.rules import qcgd
+from quids_amd.state import HostState
+
+from helpers import assert_states_identical, qcgd_initial
+
+pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def _device_filled(leave):
+    """Takes device memory until about `leave` bytes are left."""
+    q.default_context().trim()
+    held = []
+    try:
+        for _ in range(64):
+            free = torch.cuda.mem_get_info()[0]
+            if free < leave + (32 << 20):
+                break
+            held.append(torch.empty(min(free - leave, 32 << 30), dtype=torch.uint8, device="cuda"))
+        yield
+    finally:
+        held.clear()
+        torch.cuda.empty_cache()
+
+
+# output states whose offsets could not be allocated (their other buffers are
+# the smallest ones): as many survivors as those hold, more, and none
+def test_output_states_after_a_failed_upload():
+    n = 48 << 20  # objects of no bytes: 384 MB of offsets
+    outs = [q.it_t() for _ in range(3)]
+    with _device_filled(256 << 20):
+        for out in outs:
+            with pytest.raises(QuidsError) as e:
+                out.upload(HostState(np.zeros(0, np.uint8), np.zeros(n + 1, np.uint64), np.zeros(n, np.uint32),
+                                     np.zeros(n, np.complex128)))
+            assert e.value.code == QD_ERR_OOM
+    rule, old = qcgd.erase_create(0.8, 0.3), q.tolerance
+    for out, (nodes, tolerance) in zip(outs, [(3, 1e-30), (12, 1e-30), (12, 2.0)]):
+        hs = qcgd_initial(nodes, 42)
+        a = q.it_t()
+        a.upload(hs)
+        q.tolerance = tolerance
+        try:
+            q.simulate(a, rule, out, None, q.UINT64_MAX)
+        finally:
+            q.tolerance = old
+        ref, _ = orc.simulate(hs, rule, tolerance=tolerance)
+        assert_states_identical(out.download(), ref, f"{nodes} nodes, tolerance {tolerance}")
+        a.close()
+        out.close()

@@ -28,3 +28,12 @@ def test_places_of_objects(lib, size, align):
         assert at[k] == want
         want += (s + align - 1) // align * align
     assert end == want
+
+
+# bytes of a state's begin, size and magnitude buffers (0: no buffer), and the objects they hold
+@pytest.mark.parametrize("bytes_of,objects", [((0, 0, 0), 0), ((0, 256, 256), 0), ((8, 256, 256), 0), ((256, 0, 256), 0),
+                                              ((256, 256, 0), 0), ((24, 256, 256), 2), ((256, 256, 256), 16),
+                                              ((1 << 40, 12, 1 << 40), 3), ((8 * 101, 400, 1600), 100)])
+def test_room_of_a_state(lib, bytes_of, objects):
+    lib.host_state_room.restype = ctypes.c_uint64
+    assert lib.host_state_room(*map(ctypes.c_uint64, bytes_of)) == objects
