@@ -83,7 +83,8 @@ enum : u32 {
     LEAN_BIG = 4u,      // more candidates than there is room for
     LEAN_BUCKET = 8u,   // a bucket that the main dedup kernel hands back
     LEAN_SPILL = 32u,   // a bucket beyond its capacity (ERR_SPILL1's bit)
-    LEAN_SELECT = 64u   // more tied keys than one block takes, or a subnormal threshold
+    LEAN_SELECT = 64u,  // more tied keys than one block takes, or a subnormal threshold
+    LEAN_ROOM = 128u    // (the host's) a buffer does not fit the free memory
 };
 // Kernels that can stop the step, in launch order.  Each sets its own word,
 // and a kernel looks only at the words of the kernels before it, so that

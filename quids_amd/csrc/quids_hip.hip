@@ -2279,8 +2279,8 @@ static bool lean_allowed(qd_ctx *ctx, const SelKey &sk) {
 // them when the host knows (C != 0), else what the scan found.  One wait, at
 // the end; a second one when the output state had to grow.
 template <int KIND>
-static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule &rule, const LeanArea &la, u64 room, u64 C,
-                     u64 nitems, u64 max_obj, const qd_params &prm, qd_state *out, qd_step_stats &st, LeanEnd &le) {
+static int lean_run(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule &rule, const LeanArea &la, u64 room, u64 C,
+                    u64 nitems, u64 max_obj, const qd_params &prm, qd_state *out, qd_step_stats &st, LeanEnd &le) {
     hipStream_t s = ctx->stream;
     u64 *a = ctx->lean.as<u64>();
     LeanPlan *lp = reinterpret_cast<LeanPlan *>(a);
@@ -2314,6 +2314,8 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
     // to slots, which the generate clears (else it takes the entries' place
     // once the dedup has read them)
     const bool all = !keys && !items;
+    const u64 nchunk = items ? (nitems + kGenThreads - 1) / kGenThreads : 0;
+    if (items) QD_TRY(ensure_relieved(ctx, ctx->cpar, nchunk * sizeof(u64)));
     u32 *slotof = all ? ctx->ukey.as<u32>() : ctx->ebuf1.as<u32>();
     u64 *nhist = a + la.nhist, *hist2 = a + la.hist2, *cnt1 = a + la.cnt1;
     if (C) {  // a fresh state: pooled buffers of about the size that a truncated step's survivors need
@@ -2329,8 +2331,6 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
 
     prof_begin(ctx, QD_PHASE_GENERATE);
     if (items) {
-        const u64 nchunk = (nitems + kGenThreads - 1) / kGenThreads;
-        QD_TRY(ensure_relieved(ctx, ctx->cpar, nchunk * sizeof(u64)));
         hipLaunchKernelGGL(k_chunk_parent, dim3(grid_for(nchunk)), dim3(256), 0, s, ctx->wb.as<u64>(), P.n, nchunk,
                            ctx->cpar.as<u64>());
         hipLaunchKernelGGL((k_generate_scatter<KIND == QD_RULE_HADAMARD ? QD_RULE_QCGD_COIN : KIND, false>),
@@ -2444,6 +2444,21 @@ static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule 
     return QD_OK;
 }
 
+// lean_run; a step whose buffers do not fit the free memory (up to 240 bytes a
+// candidate here) goes on on the host-driven path, which makes do with 150 or
+// less and runs in hash-range passes when those do not fit either.
+template <int KIND>
+static int lean_tail(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule &rule, const LeanArea &la, u64 room, u64 C,
+                     u64 nitems, u64 max_obj, const qd_params &prm, qd_state *out, qd_step_stats &st, LeanEnd &le) {
+    const int rc = lean_run<KIND>(ctx, P, in_bytes, rule, la, room, C, nitems, max_obj, prm, out, st, le);
+    if (rc != QD_ERR_OOM) return rc;
+    QD_HIP(hipStreamSynchronize(ctx->stream));  // (the scan's report)
+    prof_collect(ctx);
+    le = LeanEnd{};
+    le.stop = LEAN_ROOM;
+    return QD_OK;
+}
+
 template <int KIND, bool BATCH>
 static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, const qd_rule &rule, Batch *bt,
                      qd_state *out, qd_symbolic *sy, u64 max_obj, const qd_params &prm, qd_step_stats &st) {
@@ -2547,8 +2562,11 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     QD_TRY(ensure_relieved(ctx, ctx->ctab, kLeanTab * sizeof(u64)));
     i32 *delta = nullptr;
     if (lean && KIND == QD_RULE_QCGD_SPLIT_MERGE) {
-        QD_TRY(ensure_relieved(ctx, ctx->delta, (sm_delta_base(in_bytes) + 64) * sizeof(i32)));
-        delta = ctx->delta.as<i32>();
+        const int rc = ensure_relieved(ctx, ctx->delta, (sm_delta_base(in_bytes) + 64) * sizeof(i32));
+        if (rc && rc != QD_ERR_OOM) return rc;
+        delta = ctx->delta.as<i32>();  // (null if it does not fit: the host-driven path does without it)
+        lean = delta != nullptr;
+        if (!lean) room = 0;
     }
     hipLaunchKernelGGL(k_lean_clear, dim3(grid_for(la.words, 256, 256)), dim3(256), 0, s, ctx->lean.as<u64>(), la.words,
                        counters, u64(64));

@@ -13,7 +13,7 @@ from quids_amd._abi import QD_ERR_OOM, QuidsError
 from quids_amd.rules import qcgd
 from quids_amd.state import HostState
 
-from helpers import assert_states_identical, qcgd_initial
+from helpers import assert_states_identical, qcgd_initial, sparse_graph
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +60,22 @@ def test_output_states_after_a_failed_upload():
         assert_states_identical(out.download(), ref, f"{nodes} nodes, tolerance {tolerance}")
         a.close()
         out.close()
+
+
+# 15 graphs of 20 free nodes each: 1.6e7 children, of which a device-driven
+# step would hold 3.8 GB at once
+def test_large_step_on_a_nearly_full_device():
+    hs = HostState.from_objects([sparse_graph(22, (), (k,)) for k in range(15)])
+    rule = qcgd.erase_create(0.8, 0.3)
+    a = q.it_t()
+    a.upload(hs)
+    out = []
+    for left in (0, 2800 << 20):
+        b = q.it_t()
+        with _device_filled(left) if left else contextlib.nullcontext():
+            st = q.simulate(a, rule, b, None, 1000)
+        assert st["num_candidates"] == 15 << 20 and bool(st["reserved"] & 4) == bool(left)
+        out.append(b.download())
+        b.close()
+    a.close()
+    assert_states_identical(out[1], out[0], "nearly full")
