@@ -2552,8 +2552,8 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     const u64 lean_max = fast && ctx->tune.chunk_log2 ? std::min<u64>(kLeanMax, 1ull << ctx->tune.chunk_log2) : kLeanMax;
     if (room > lean_max) room = 0;
     // (a device-driven step keeps to buffers of its own: views into the slab
-    // of the hash-range passes go when an allocation does not fit beside it,
-    // or the step falls back)
+    // of the hash-range passes go with it when an allocation does not fit
+    // beside it, the step falls back or ends)
     if (lean)
         for (DBuf *b : {&ctx->ebuf2, &ctx->ukey})
             if (b->view) b->release();
@@ -2659,6 +2659,7 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
         QD_TRY(lean_tail<KIND>(ctx, P, in_bytes, rule, la, C, C, nitems, max_obj, prm, out, st, le));
     }
     if (le.done) {
+        release_range_cache(ctx);  // one pass, as below: the slab's memory goes back to the device
         u32 b1, b2;
         dedup_layout(C, ctx->tune, b1, b2);
         st.dedup_levels = (b1 ? 1 : 0) + (b2 ? 1 : 0);

@@ -79,3 +79,26 @@ def test_large_step_on_a_nearly_full_device():
         b.close()
     a.close()
     assert_states_identical(out[1], out[0], "nearly full")
+
+
+def test_small_step_gives_up_the_hash_range_buffers():
+    ctx = q.default_context()
+    old = ctx.get_tuning()
+    ctx.trim()
+    hs = HostState.from_objects([sparse_graph(22, (), (k,)) for k in range(2)])
+    rule = qcgd.erase_create(0.8, 0.3)
+    a, b = q.it_t(), q.it_t()
+    a.upload(hs)
+    ctx.set_tuning(chunk_log2=20)
+    try:
+        assert q.simulate(a, rule, b, None, 1000)["reserved"] & 4
+    finally:
+        ctx.set_tuning(chunk_log2=old["chunk_log2"])
+    ranged = torch.cuda.mem_get_info()[0]
+    a.upload(qcgd_initial(6, 42))
+    q.simulate(a, rule, b, None, 1000)
+    # (a slab of the tags, the pool and passes of 2^20 candidates: more than
+    # what the step asked for itself)
+    assert torch.cuda.mem_get_info()[0] > ranged
+    a.close()
+    b.close()
