@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
+
 #include "qd_rules.hpp"
 
 namespace qd {
@@ -99,9 +101,11 @@ struct LeanPlan {
     u64 K, bytes;      // survivors and their padded bytes
     u32 b1, b2;        // bits of the radix passes
     u32 d1;            // select: the first digit
-    u32 ticket[3];     // next tiles of the look-back kernels; blocks of the generate that ended
+    alignas(8) u32 ticket[3];  // next tiles of the look-back kernels; blocks of the generate that ended
     u32 stop[LEAN_EMIT];  // LEAN_* by kernel (the dedup's: counters 5 and 6)
 };
+// (the first two are cleared as one word when the order runs again)
+static_assert(offsetof(LeanPlan, ticket) % sizeof(u64) == 0, "the tickets of the look-back kernels share a u64");
 // What the last kernel reports to the host (pinned memory).
 struct LeanReport {
     u64 U, K, bytes;
