@@ -1,4 +1,4 @@
-"""Plain integer arithmetic of the library (tests/cpp/host_checks.cpp), on the CPU."""
+"""Plain host code of the library (tests/cpp/host_checks.cpp), on the CPU."""
 import ctypes
 import os
 import subprocess
@@ -37,3 +37,15 @@ def test_places_of_objects(lib, size, align):
 def test_room_of_a_state(lib, bytes_of, objects):
     lib.host_state_room.restype = ctypes.c_uint64
     assert lib.host_state_room(*map(ctypes.c_uint64, bytes_of)) == objects
+
+
+# buffers that the pool keeps: those that the device is known to have finished
+# with, of 64 KB to half its 4 GiB, the newest that fit
+@pytest.mark.parametrize("n,failing,size,kept", [(1, 0, 1 << 20, 1), (1, 1, 1 << 20, 0), (5, 2, 1 << 20, 3),
+                                                 (3, 0, 1 << 15, 0), (3, 0, 3 << 30, 0), (6, 0, 1 << 30, 4),
+                                                 (70, 0, 1 << 20, 64)])
+def test_pooled_buffers(lib, n, failing, size, kept):
+    lib.host_pool_give.restype = ctypes.c_uint64
+    freed = ctypes.c_uint64()
+    assert lib.host_pool_give(*map(ctypes.c_uint64, (n, failing, size)), ctypes.byref(freed)) == kept * size
+    assert freed.value == n - kept
