@@ -2206,6 +2206,7 @@ struct LeanEnd {
     bool done = false;  // the output state is complete
     u32 stop = 0;       // else why not (LEAN_*)
     u64 U = 0;
+    u32 levels = 0;  // radix passes of its dedup
 };
 
 // The device-driven step takes plain |m|^2 keys and the default layout; a
@@ -2354,6 +2355,7 @@ static int lean_run(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule &
         prof_collect(ctx);
         le.stop = rep->stop;
         le.U = rep->U;
+        le.levels = (rep->b1 ? 1 : 0) + (rep->b2 ? 1 : 0);
         if (rep->stop) return QD_OK;
         if (rep->fits) break;
         if (attempt) return fail(QD_ERR_HIP, "device-driven step: the output does not fit the room made for it");
@@ -2601,9 +2603,7 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     }
     if (le.done) {
         release_range_cache(ctx);  // one pass, as below: the slab's memory goes back to the device
-        u32 b1, b2;
-        dedup_layout(C, ctx->tune, b1, b2);
-        st.dedup_levels = (b1 ? 1 : 0) + (b2 ? 1 : 0);
+        st.dedup_levels = le.levels;
         if (st.num_survivors == 0) return finish_empty();
         if (sy) {
             sy->num_object = C;
@@ -2743,6 +2743,7 @@ static int step_impl(qd_ctx *ctx, const Parents &P, u64 in_bytes, u64 in_mem, co
     u64 U;
     phase_mark(ctx, PH_COLL_PREP);
     if (deduped) {
+        st.dedup_levels = le.levels;
         UH = H0;
         UR = UH + C;
         UM = reinterpret_cast<double2 *>(UR + C);
