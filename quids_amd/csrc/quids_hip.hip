@@ -170,6 +170,7 @@ struct DBuf {
             if (e != hipSuccess) {
                 (void)hipGetLastError();
                 p = nullptr;
+                nominal = 0;
                 size_t freeb = 0, totalb = 0;
                 (void)hipMemGetInfo(&freeb, &totalb);
                 return fail(QD_ERR_OOM, "hipMalloc of " + std::to_string(bytes) + " bytes failed (device free " +

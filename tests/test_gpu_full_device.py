@@ -102,3 +102,28 @@ def test_small_step_gives_up_the_hash_range_buffers():
     assert torch.cuda.mem_get_info()[0] > ranged
     a.close()
     b.close()
+
+
+# memory-driven truncation counts what the output state holds: the same for a
+# new state and for one whose upload failed
+def test_memory_of_a_state_after_a_failed_upload():
+    n = 48 << 20
+    failed, fresh, a = q.it_t(), q.it_t(), q.it_t()
+    with _device_filled(256 << 20):
+        with pytest.raises(QuidsError):
+            failed.upload(HostState(np.zeros(0, np.uint8), np.zeros(n + 1, np.uint64), np.zeros(n, np.uint32),
+                                    np.zeros(n, np.complex128)))
+    a.upload(qcgd_initial(8, 42))
+    ctx = q.default_context()
+    old = ctx.get_tuning()
+    ctx.set_tuning(free_mem_mib=64)
+    try:
+        targets = []
+        for out in (failed, fresh):
+            ctx.trim()
+            targets.append(q.simulate(a, qcgd.split_merge(0.8, 0.3), out, None, 0)["mem_target_parents"])
+    finally:
+        ctx.set_tuning(free_mem_mib=old["free_mem_mib"])
+    assert abs(targets[0] - targets[1]) <= 1 << 10, targets  # (the failed state lacks a buffer of 256 bytes)
+    for s in (failed, fresh, a):
+        s.close()
