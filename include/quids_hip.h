@@ -132,7 +132,11 @@ int qd_ctx_synchronize(qd_ctx *ctx);
 int qd_ctx_stream(qd_ctx *ctx, void **stream);
 /* Device-side bytes currently held by the context's scratch pool. */
 int qd_ctx_scratch_bytes(qd_ctx *ctx, uint64_t *bytes);
-/* Release the context's cached scratch buffers. */
+/* Release the context's cached scratch buffers, and the state buffers that it
+ * keeps: those of closed and grown states, at most 4 GiB, stay with the context
+ * for its next states (not counted by qd_ctx_scratch_bytes; also given back
+ * when an allocation of the library does not fit).  Other allocators of the
+ * process cannot reclaim them. */
 int qd_ctx_trim(qd_ctx *ctx);
 
 /* Phase timing of simulate() with HIP events on the context's stream (the

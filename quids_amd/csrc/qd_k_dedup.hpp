@@ -527,8 +527,9 @@ __global__ __launch_bounds__(T) void k_dedup(const Entry *E, u64 rstride, const 
         }
         const u32 W = wcount;  // uniform
         if (W && W <= u32(kWave)) {
-            // one wavefront: bitonic sort in registers, then the segmented
-            // pairwise tree by shuffles; no block barrier until the results
+            // one wavefront: each lane ranks its entry by counting the smaller
+            // ones, then the segmented pairwise tree by shuffles; no block
+            // barrier until the results
             if (threadIdx.x < kWave) {
                 const u32 l = threadIdx.x;
                 const bool valid = l < W;

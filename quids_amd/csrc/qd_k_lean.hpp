@@ -9,13 +9,14 @@
 // it, about 5 us of device idle time per launch and 15-20 us per wait
 // (a 12-node split_merge step of 1.4e6 candidates: 91 launches, 0.51 ms of
 // kernels in 0.73 ms; a 6-node step of 3e3: 42 launches, 0.15 ms in 0.25 ms).
-// Driven from the device they take 16 and 14 launches and one or two waits:
-// two 6-node iterations went from 1.22 to 0.53 ms, four truncated 9-node ones
-// from 3.33 to 1.26 ms, the split_merge step from 0.83 to 0.53 ms, a 12-node
-// erase_create step of 6e6 candidates from 0.96 to 0.68 ms.  Fixed grids cost
-// little: a block with nothing to do exits within the launch overhead.  Larger
-// steps (beyond kLeanMax) spend under 2 % on launches and waits and keep
-// buffers sized for their own counts.
+// Driven from the device they take 15 and 11 launches and one or two waits.
+// With that, shorter kernels and pooled state buffers, two 6-node iterations
+// went from 1.25 to 0.42 ms, four truncated 9-node ones from 3.36 to 1.03 ms,
+// a 12-node split_merge step of 2.9e6 candidates from 0.82 to 0.46 ms, an
+// erase_create one of 6e6 from 0.95 to 0.62 ms.  Fixed grids cost little: a
+// block with nothing to do exits within the launch overhead.  Larger steps
+// (beyond kLeanMax) spend under 2 % on launches and waits and keep buffers
+// sized for their own counts.
 #include <hip/hip_runtime.h>
 
 #include "qd_device.hpp"
@@ -487,7 +488,9 @@ __global__ __launch_bounds__(1024) void k_sel_finish(const SelItem *S, u32 ns, u
 // step of 1.4e6 candidates and 2e4 survivors.  Bound by a tile's chain of
 // dependent reads (ticket, slots, parent search, size, look-backs), so a tile
 // has 1024 threads: where every candidate survives, 256 of them took it in 16
-// rounds (2^17 hadamard children 21 us, now 13).
+// rounds (2^17 hadamard children 21 us, now 13).  Byte offsets are 64-bit, in
+// the registers of the thread that sums a run of the list, which writes them
+// (the same time as a 32-bit list in LDS, which 4096 survivors of 1 MiB pass).
 // ---------------------------------------------------------------------------
 constexpr u32 kEmitTile = 4096;
 constexpr u32 kEmitThreads = 1024;

@@ -28,8 +28,9 @@ struct LoadPopc {
 };
 
 // ---------------------------------------------------------------------------
-// decoupled look-back: the exclusive prefix of a tile's aggregate over the
-// tiles before it.  desc[t] = status | epoch | value of VB bits: words of an
+// decoupled look-back (the method of Merrill and Garland, "Single-pass
+// Parallel Prefix Scan with Decoupled Look-back", 2016): the exclusive prefix
+// of a tile's aggregate over the tiles before it.  desc[t] = status | epoch | value of VB bits: words of an
 // earlier launch carry another epoch and read as not there yet, so a buffer
 // is cleared when it is made and when the epochs wrap, not for every scan
 // (VB = 62: no epochs, cleared for every scan).

@@ -1700,11 +1700,13 @@ static int range_step(qd_ctx *ctx, const Parents &P, u64 in_bytes, const qd_rule
     QD_TRY(carve(ctx->rpart[0], std::max<u64>(u64(ngroups) * gbytes, nmax * sizeof(Entry))));
     std::vector<u32> rc(u64(ngroups) * gr);
     bool l2_exact = false;  // second pass with exact offsets (after a spill)
-    // A group has at most 128 first-level buckets (nb1 / 8): several
-    // workgroups each, which take their places in a sub-bucket from one
-    // counter (one workgroup each left half the CUs idle: 152 us a group of
-    // 7.3e6 candidates, now 107); beyond 2^8 sub-buckets a chunk would go to
-    // memory for a place of every few entries.
+    // A group of an eighth of a pass has at most 128 first-level buckets
+    // (nb1 / 8, up to 1024 where passes are small and groups fewer): with
+    // fewer buckets than workgroups fit the chip (kL2Grid), several workgroups
+    // each, which take their places in a sub-bucket from one counter (one
+    // workgroup each left half the CUs idle: 152 us a group of 7.3e6
+    // candidates, now 107); beyond 2^8 sub-buckets a chunk would go to memory
+    // for a place of every few entries.
     const u32 l2_parts = b2 && b2 <= 8 ? u32(std::max<u64>(kL2Grid / gbk, 1)) : 1;
     tl[4] = wall_ms();
     phase_mark(ctx, PH_COLL_INSERT);
